@@ -192,6 +192,34 @@ int jo_fused_qk_norm_rope_3d_grid_kstage(void* q, void* k, void* k_stage, int64_
                                          float source_id, void* stream);
 
 /* ------------------------------------------------------------------------
+ * fused_qk_norm_rope_3d_paired (and, with k_stage, _paired_kstage) as the DiT
+ * calls it: fp32 rotation tables, strided q / k sources and destinations of
+ * their own, in one launch.
+ *   q_out = rope(rmsnorm(q)), k_out likewise, with the tables' values rounded
+ *   to bf16 first: bit for bit the results of the paired op on contiguous
+ *   copies of q, k and bf16 copies of the tables' pair values.
+ * Replaces the caller's glue around the paired op
+ *   (deploy/xvideo/models/dit/sgl_fused_ops.py:73-94: .contiguous() of q and
+ *    k, the tables sliced, copied and cast).
+ * cos, sin: fp32, row n at n * table_row_stride elements, pair p's value at
+ * element p * table_step (1: [seq_len, head_dim/2]; 2: [seq_len, head_dim],
+ * each value held twice); 16-byte aligned, the row stride a multiple of 4.
+ * q_out / k_out: bf16 rows with their own batch and token strides, each
+ * either its own source (same pointer and strides: in place) or overlapping
+ * neither q nor k. k_stage (optional, null: none): as for _paired_kstage.
+ * ------------------------------------------------------------------------ */
+int jo_fused_qk_norm_rope_3d_tables(const void* q, const void* k, void* q_out, void* k_out,
+                                    void* k_stage, int64_t batch, int64_t seq_len,
+                                    int64_t num_heads, int64_t head_dim, int64_t q_batch_stride,
+                                    int64_t q_token_stride, int64_t k_batch_stride,
+                                    int64_t k_token_stride, int64_t q_out_batch_stride,
+                                    int64_t q_out_token_stride, int64_t k_out_batch_stride,
+                                    int64_t k_out_token_stride, int64_t stage_batch_stride,
+                                    int64_t stage_token_stride, float eps, const void* q_weight,
+                                    const void* k_weight, const float* cos, const float* sin,
+                                    int64_t table_row_stride, int32_t table_step, void* stream);
+
+/* ------------------------------------------------------------------------
  * Grid-mode QK norm + RoPE that writes the rotated K straight into a frame
  * ring buffer: q is updated in place, k is only read, and the rotated head
  * vectors of k for frame f go to cache frame slot (slot_start + f) % cache_slots,

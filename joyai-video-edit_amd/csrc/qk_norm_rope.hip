@@ -5,9 +5,18 @@
 // load covers 512 contiguous elements = 512/D heads), so one token's
 // rotation coefficients are fetched or computed once and reused for every
 // head of q and k. Each head's sum of squares reduces over its D/8 lanes with
-// DPP row operations. Three modes share the kernel:
+// DPP row operations. Four modes share the kernel:
 //   TABLE  coefficients read from bf16 cos/sin [seq_len, D/2] tables
 //          (drop-in for fused_qk_norm_rope_3d_paired);
+//   TAB32  coefficients read from the fp32 tables that the DiT hands its
+//          caller and rounded to bf16 in registers, rows written to a
+//          destination of their own (which may be the source). Bound by HBM:
+//          the copies of q and k, the four table kernels and the TABLE pass
+//          that it stands for moved the rows twice and waited on each other's
+//          launches ([1, 3120, 32, 128] slices of a packed qkv 50.4 -> 19.3 us,
+//          5.4 TB/s of the bytes needed, 0.99 of a 256 MiB copy's rate; with
+//          the K stage, [1, 1560, 32, 128], 37.1 -> 14.5 us; nontemporal
+//          instead of written-through row stores: level);
 //   GRID   coefficients computed in registers from the token's (t, h, w)
 //          grid position: each lane evaluates sincos for D/128 (min 1) pairs
 //          and the wave redistributes them with ds_bpermute;
@@ -25,6 +34,7 @@ constexpr int kMaxPairs = 128;  // head_dim 256
 constexpr int kTable = 0;
 constexpr int kGrid = 1;
 constexpr int kKvCache = 2;
+constexpr int kTable32 = 3;
 
 struct QKArgs {
   void* q;
@@ -53,6 +63,13 @@ struct QKArgs {
   // compiles to loads from the kernel-argument segment). No device copy, so a
   // grid launch needs no setup and captures into a HIP graph as it is.
   float freqs[2 * kMaxPairs];
+  // TAB32: q's destination, fp32 table rows tab_rs elements apart with a
+  // pair's value at every tab_step-th element (1: [L, D/2]; 2: [L, D], each
+  // value held twice).
+  void* qout;
+  int64_t qo_bs, qo_ts;
+  int64_t tab_rs;
+  int tab_step;
 };
 
 // sin and cos of an fp32 angle a. For |a| <= 65536: Cody-Waite reduction by
@@ -173,7 +190,7 @@ __global__ __launch_bounds__(kBlock) void qk_norm_rope_kernel(const QKArgs a) {
   // Destination token of the rotated k (grid modes: frame ring slot).
   int64_t kdst_tok = n;
   int f = 0, rr = 0;
-  if constexpr (MODE != kTable) {
+  if constexpr (MODE == kGrid || MODE == kKvCache) {
     const int frame_tokens = a.grid_h * a.grid_w;
     f = static_cast<int>(fdiv(static_cast<uint32_t>(n), a.fd_frame));
     rr = n - f * frame_tokens;
@@ -187,16 +204,18 @@ __global__ __launch_bounds__(kBlock) void qk_norm_rope_kernel(const QKArgs a) {
   const char* krow = static_cast<const char*>(a.k) + (b * a.k_bs + n * a.k_ts) * 2;
   char* kdst = static_cast<char*>(a.kout) + (b * a.o_bs + kdst_tok * a.o_ts) * 2;
   char* kstg = STAGE ? static_cast<char*>(a.kstage) + (b * a.s_bs + n * a.s_ts) * 2 : nullptr;
+  char* qdst = qrow;
+  if constexpr (MODE == kTable32) qdst = static_cast<char*>(a.qout) + (b * a.qo_bs + n * a.qo_ts) * 2;
   const char* src[NS];
   char* dst[NS];
   const char* wsrc[NS];
   if constexpr (NS == 2) {
-    src[0] = qrow; dst[0] = qrow; wsrc[0] = static_cast<const char*>(a.qw);
+    src[0] = qrow; dst[0] = qdst; wsrc[0] = static_cast<const char*>(a.qw);
     src[1] = krow; dst[1] = kdst; wsrc[1] = static_cast<const char*>(a.kw);
   } else {
     const bool is_k = (part & 1) != 0;  // wave-uniform
     src[0] = is_k ? krow : qrow;
-    dst[0] = is_k ? kdst : qrow;
+    dst[0] = is_k ? kdst : qdst;
     wsrc[0] = static_cast<const char*>(is_k ? a.kw : a.qw);
   }
   // Head groups (512 elements each) this wave handles: all of its tensor's,
@@ -209,11 +228,21 @@ __global__ __launch_bounds__(kBlock) void qk_norm_rope_kernel(const QKArgs a) {
 
   // 1. Parameter loads: rotation table row or frequencies, weights.
   u32x2 cw, sw;
+  u32x4 c32[2], s32[2];
   float fq[K], fr[K];
   if constexpr (MODE == kTable) {
     const int64_t off = (static_cast<int64_t>(n) * P + 4 * pl) * 2;
     cw = *reinterpret_cast<const u32x2*>(static_cast<const char*>(a.cos) + off);
     sw = *reinterpret_cast<const u32x2*>(static_cast<const char*>(a.sin) + off);
+  } else if constexpr (MODE == kTable32) {
+    // Pairs 4*pl .. 4*pl+3: 16 or 32 bytes of a row (with a step of 1 the
+    // second load repeats the first, so no load is behind a branch).
+    const int64_t off = n * a.tab_rs + 4 * pl * a.tab_step;
+    const int second = 4 * (a.tab_step - 1);
+    c32[0] = ld16(static_cast<const float*>(a.cos) + off);
+    c32[1] = ld16(static_cast<const float*>(a.cos) + off + second);
+    s32[0] = ld16(static_cast<const float*>(a.sin) + off);
+    s32[1] = ld16(static_cast<const float*>(a.sin) + off + second);
   } else {
 #pragma unroll
     for (int k = 0; k < K; ++k) {
@@ -254,6 +283,17 @@ __global__ __launch_bounds__(kBlock) void qk_norm_rope_kernel(const QKArgs a) {
   if constexpr (MODE == kTable) {
     c[0] = bf16_lo(cw.x); c[1] = bf16_hi(cw.x); c[2] = bf16_lo(cw.y); c[3] = bf16_hi(cw.y);
     s[0] = bf16_lo(sw.x); s[1] = bf16_hi(sw.x); s[2] = bf16_lo(sw.y); s[3] = bf16_hi(sw.y);
+  } else if constexpr (MODE == kTable32) {
+    const bool wide = a.tab_step == 2;
+    auto four = [&](const u32x4 (&t)[2], float (&o)[4]) {
+      const float v[8] = {elem<F32>(t[0], 0), wide ? elem<F32>(t[0], 2) : elem<F32>(t[0], 1),
+                          wide ? elem<F32>(t[1], 0) : elem<F32>(t[0], 2),
+                          wide ? elem<F32>(t[1], 2) : elem<F32>(t[0], 3), 0.f, 0.f, 0.f, 0.f};
+      const u32x4 b = pack<BF16>(v);  // the bf16 tables of the paired op
+      o[0] = bf16_lo(b.x); o[1] = bf16_hi(b.x); o[2] = bf16_lo(b.y); o[3] = bf16_hi(b.y);
+    };
+    four(c32, c);
+    four(s32, s);
   } else {
     const int hh = static_cast<int>(fdiv(static_cast<uint32_t>(rr), a.fd_gw));
     const int ww = rr - hh * a.grid_w;
@@ -364,7 +404,7 @@ int launch_qk(const QKArgs& args, int head_dim, hipStream_t stream, const char* 
   QKArgs a = args;
   a.fd_seq = make_fastdiv(static_cast<uint32_t>(a.seq_len));
   a.fd_row = make_fastdiv(static_cast<uint32_t>(a.row_elems));
-  if (MODE != kTable) {
+  if (MODE == kGrid || MODE == kKvCache) {
     a.fd_gw = make_fastdiv(static_cast<uint32_t>(a.grid_w));
     a.fd_frame = make_fastdiv(static_cast<uint32_t>(a.grid_h) * static_cast<uint32_t>(a.grid_w));
   }
@@ -523,6 +563,51 @@ int qk_grid(const char* op, void* q, void* k, void* k_stage, int64_t batch, int6
 
 }  // namespace
 }  // namespace jo
+
+extern "C" int jo_fused_qk_norm_rope_3d_tables(
+    const void* q, const void* k, void* q_out, void* k_out, void* k_stage, int64_t batch,
+    int64_t seq_len, int64_t num_heads, int64_t head_dim, int64_t q_batch_stride,
+    int64_t q_token_stride, int64_t k_batch_stride, int64_t k_token_stride,
+    int64_t q_out_batch_stride, int64_t q_out_token_stride, int64_t k_out_batch_stride,
+    int64_t k_out_token_stride, int64_t stage_batch_stride, int64_t stage_token_stride, float eps,
+    const void* q_weight, const void* k_weight, const float* cos, const float* sin,
+    int64_t table_row_stride, int32_t table_step, void* stream) {
+  const char* op = "fused_qk_norm_rope_3d_tables";
+  int st = check_qk(op, q, k, batch, seq_len, num_heads, head_dim, q_batch_stride, q_token_stride,
+                    k_batch_stride, k_token_stride, q_weight, k_weight);
+  if (st != JO_OK) return st;
+  const int64_t row = num_heads * head_dim;
+  JO_REQUIRE(q_out_token_stride >= row && k_out_token_stride >= row && q_out_batch_stride >= 0 &&
+                 k_out_batch_stride >= 0 && q_out_token_stride % 8 == 0 &&
+                 k_out_token_stride % 8 == 0 && q_out_batch_stride % 8 == 0 &&
+                 k_out_batch_stride % 8 == 0,
+             "%s: bad output strides", op);
+  JO_REQUIRE(table_step == 1 || table_step == 2, "%s: table_step must be 1 or 2", op);
+  JO_REQUIRE(table_row_stride >= head_dim / 2 * table_step && table_row_stride % 4 == 0,
+             "%s: table rows must cover their pairs and keep 16-byte alignment", op);
+  if (batch * seq_len == 0) return JO_OK;
+  JO_REQUIRE(q_out && k_out && aligned(q_out, 16) && aligned(k_out, 16),
+             "%s: outputs must be 16-byte aligned pointers", op);
+  JO_REQUIRE(cos && sin && aligned(cos, 16) && aligned(sin, 16),
+             "%s: cos/sin must be 16-byte aligned pointers", op);
+  if (k_stage && (st = check_stage(op, k_stage, stage_batch_stride, stage_token_stride, num_heads,
+                                   head_dim)) != JO_OK)
+    return st;
+  QKArgs a{};
+  a.q = const_cast<void*>(q); a.k = k; a.kout = k_out; a.qout = q_out;
+  a.q_bs = q_batch_stride; a.q_ts = q_token_stride;
+  a.k_bs = k_batch_stride; a.k_ts = k_token_stride;
+  a.qo_bs = q_out_batch_stride; a.qo_ts = q_out_token_stride;
+  a.o_bs = k_out_batch_stride; a.o_ts = k_out_token_stride;
+  a.kstage = k_stage; a.s_bs = stage_batch_stride; a.s_ts = stage_token_stride;
+  a.tokens = batch * seq_len; a.seq_len = static_cast<int>(seq_len);
+  a.row_elems = static_cast<int>(row); a.eps = eps;
+  a.qw = q_weight; a.kw = k_weight; a.cos = cos; a.sin = sin;
+  a.tab_rs = table_row_stride; a.tab_step = table_step;
+  hipStream_t hs = static_cast<hipStream_t>(stream);
+  return k_stage ? launch_qk<kTable32, true>(a, static_cast<int>(head_dim), hs, op)
+                 : launch_qk<kTable32>(a, static_cast<int>(head_dim), hs, op);
+}
 
 extern "C" int jo_fused_qk_norm_rope_3d_paired(void* q, void* k, int64_t batch, int64_t seq_len,
                                                int64_t num_heads, int64_t head_dim,

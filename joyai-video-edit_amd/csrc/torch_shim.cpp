@@ -416,6 +416,66 @@ void fused_qk_norm_rope_3d_paired_kstage(torch::Tensor& q, torch::Tensor& k,
                "fused_qk_norm_rope_3d_paired_kstage");
 }
 
+namespace {
+// fp32 rotation tables [L, D/2] or [L, D] (each value held twice) as the
+// tables entry point reads them; returns their element step.
+int32_t check_tables32(const torch::Tensor& cos, const torch::Tensor& sin, const QKGeom& g) {
+  JO_CHECK_CUDA(cos);
+  JO_CHECK_CUDA(sin);
+  JO_CHECK_DTYPE(cos, torch::kFloat32);
+  JO_CHECK_DTYPE(sin, torch::kFloat32);
+  TORCH_CHECK(cos.dim() == 2 && sin.sizes() == cos.sizes() && cos.size(0) == g.seq_len &&
+                  (cos.size(1) == g.head_dim || cos.size(1) == g.head_dim / 2),
+              "cos/sin must be [seq_len, head_dim] or [seq_len, head_dim/2]");
+  TORCH_CHECK(cos.stride(1) == 1 && sin.stride(1) == 1 && row_stride(cos) == row_stride(sin),
+              "cos/sin must have contiguous rows, equally far apart");
+  return cos.size(1) == g.head_dim ? 2 : 1;
+}
+}  // namespace
+
+// The paired op on strided q / k with the DiT's fp32 tables: new contiguous
+// rotated q and k (inputs untouched).
+std::tuple<torch::Tensor, torch::Tensor> fused_qk_norm_rope_3d_tables(
+    const torch::Tensor& q, const torch::Tensor& k, int64_t seq_len, int64_t num_heads, double eps,
+    const torch::Tensor& q_weight, const torch::Tensor& k_weight, const torch::Tensor& cos,
+    const torch::Tensor& sin) {
+  const QKGeom g = check_qk_views(q, k, seq_len, num_heads, q_weight, k_weight);
+  const int32_t step = check_tables32(cos, sin, g);
+  const c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(q.device());
+  const int64_t tok = g.num_heads * g.head_dim;
+  auto q_out = torch::empty(q.sizes(), q.options());
+  auto k_out = torch::empty(k.sizes(), k.options());
+  check_status(jo_fused_qk_norm_rope_3d_tables(
+                   q.data_ptr(), k.data_ptr(), q_out.data_ptr(), k_out.data_ptr(), nullptr,
+                   g.batch, g.seq_len, g.num_heads, g.head_dim, g.q_bs, g.q_ts, g.k_bs, g.k_ts,
+                   g.seq_len * tok, tok, g.seq_len * tok, tok, 0, 0, static_cast<float>(eps),
+                   q_weight.data_ptr(), k_weight.data_ptr(), cos.data_ptr<float>(),
+                   sin.data_ptr<float>(), row_stride(cos), step, current_stream(q)),
+               "fused_qk_norm_rope_3d_tables");
+  return {q_out, k_out};
+}
+
+// fused_qk_norm_rope_3d_paired_kstage with fp32 tables: q and k in place.
+void fused_qk_norm_rope_3d_tables_kstage(torch::Tensor& q, torch::Tensor& k,
+                                         torch::Tensor& k_stage, int64_t seq_len,
+                                         int64_t num_heads, double eps,
+                                         const torch::Tensor& q_weight,
+                                         const torch::Tensor& k_weight, const torch::Tensor& cos,
+                                         const torch::Tensor& sin) {
+  const QKGeom g = check_qk_views(q, k, seq_len, num_heads, q_weight, k_weight);
+  const int32_t step = check_tables32(cos, sin, g);
+  const auto st = stage_strides(k_stage, g);
+  if (q.numel() == 0) return;
+  const c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(q.device());
+  check_status(jo_fused_qk_norm_rope_3d_tables(
+                   q.data_ptr(), k.data_ptr(), q.data_ptr(), k.data_ptr(), k_stage.data_ptr(),
+                   g.batch, g.seq_len, g.num_heads, g.head_dim, g.q_bs, g.q_ts, g.k_bs, g.k_ts,
+                   g.q_bs, g.q_ts, g.k_bs, g.k_ts, st.first, st.second, static_cast<float>(eps),
+                   q_weight.data_ptr(), k_weight.data_ptr(), cos.data_ptr<float>(),
+                   sin.data_ptr<float>(), row_stride(cos), step, current_stream(q)),
+               "fused_qk_norm_rope_3d_tables_kstage");
+}
+
 void fused_qk_norm_rope_3d_kvcache(torch::Tensor& q, const torch::Tensor& k,
                                    torch::Tensor& k_cache, int64_t seq_len, int64_t num_heads,
                                    double eps, const torch::Tensor& q_weight,
@@ -826,6 +886,12 @@ TORCH_LIBRARY(joyomni_ops, m) {
       "int num_heads, float eps, Tensor q_weight, Tensor k_weight, Tensor freqs, int pairs_t, "
       "int pairs_h, int grid_h, int grid_w, int t0, float source_id) -> ()");
   m.def(
+      "fused_qk_norm_rope_3d_tables(Tensor q, Tensor k, int seq_len, int num_heads, float eps, "
+      "Tensor q_weight, Tensor k_weight, Tensor cos, Tensor sin) -> (Tensor, Tensor)");
+  m.def(
+      "fused_qk_norm_rope_3d_tables_kstage(Tensor! q, Tensor! k, Tensor! k_stage, int seq_len, "
+      "int num_heads, float eps, Tensor q_weight, Tensor k_weight, Tensor cos, Tensor sin) -> ()");
+  m.def(
       "fused_qk_norm_rope_3d_kvcache(Tensor! q, Tensor k, Tensor! k_cache, int seq_len, "
       "int num_heads, float eps, Tensor q_weight, Tensor k_weight, Tensor freqs, int pairs_t, "
       "int pairs_h, int grid_h, int grid_w, int t0, float source_id, int slot_start) -> ()");
@@ -859,6 +925,8 @@ TORCH_LIBRARY_IMPL(joyomni_ops, CUDA, m) {
   m.impl("sgl_per_token_quant_fp8", &joyomni_ops::sgl_per_token_quant_fp8);
   m.impl("fp8_scaled_mm", &joyomni_ops::fp8_scaled_mm);
   m.impl("fused_qk_norm_rope_3d_grid", &joyomni_ops::fused_qk_norm_rope_3d_grid);
+  m.impl("fused_qk_norm_rope_3d_tables", &joyomni_ops::fused_qk_norm_rope_3d_tables);
+  m.impl("fused_qk_norm_rope_3d_tables_kstage", &joyomni_ops::fused_qk_norm_rope_3d_tables_kstage);
   m.impl("fused_qk_norm_rope_3d_kvcache", &joyomni_ops::fused_qk_norm_rope_3d_kvcache);
   m.impl("fused_qk_norm_rope_3d_paired_kstage",
          &joyomni_ops::fused_qk_norm_rope_3d_paired_kstage);

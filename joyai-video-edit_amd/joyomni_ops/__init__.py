@@ -10,7 +10,8 @@ for device tensors only, and importing fails if the libraries are missing.
 
 New ops (no reference signature): fused_qk_norm_rope_3d_grid,
 fused_qk_norm_rope_3d_kvcache, fused_qk_norm_rope_3d_paired_kstage,
-fused_qk_norm_rope_3d_grid_kstage, fused_add_layernorm_scale_shift,
+fused_qk_norm_rope_3d_grid_kstage, fused_qk_norm_rope_3d_tables,
+fused_qk_norm_rope_3d_tables_kstage, fused_add_layernorm_scale_shift,
 rmsnorm_quant_fp8, norm_scale_shift_quant_fp8, kv_commit_rope,
 apply_rotary_emb, rmsnorm_heads, gelu_tanh_quant_fp8,
 fused_norm_scale_shift_per_sample, plus rope_freqs() to build the
@@ -53,6 +54,8 @@ __all__ = [
     "rmsnorm_heads",
     "fused_qk_norm_rope_3d_paired_kstage",
     "fused_qk_norm_rope_3d_grid_kstage",
+    "fused_qk_norm_rope_3d_tables",
+    "fused_qk_norm_rope_3d_tables_kstage",
     "gelu_tanh_quant_fp8",
     "fused_norm_scale_shift_per_sample",
 ]
@@ -184,6 +187,23 @@ def fused_qk_norm_rope_3d_grid_kstage(q, k, k_stage, seq_len, num_heads, eps, q_
     _ops.fused_qk_norm_rope_3d_grid_kstage(q, k, k_stage, seq_len, num_heads, eps, q_weight,
                                            k_weight, freqs, rope_dims[0] // 2, rope_dims[1] // 2,
                                            gh, gw, t0, float(source_id))
+
+
+def fused_qk_norm_rope_3d_tables(q, k, seq_len, num_heads, eps, q_weight, k_weight, cos, sin):
+    """fused_qk_norm_rope_3d_paired of contiguous copies of q and k with bf16 copies of
+    the tables, in one pass: returns new contiguous (q, k), the inputs untouched.
+    q/k: bf16 [B, seq_len, num_heads, D] views with contiguous heads; cos/sin:
+    fp32 [seq_len, D/2], or [seq_len, D] with each value held twice."""
+    return _ops.fused_qk_norm_rope_3d_tables(q, k, seq_len, num_heads, eps, q_weight, k_weight,
+                                             cos, sin)
+
+
+def fused_qk_norm_rope_3d_tables_kstage(q, k, k_stage, seq_len, num_heads, eps, q_weight,
+                                        k_weight, cos, sin):
+    """fused_qk_norm_rope_3d_paired_kstage with the fp32 tables of
+    fused_qk_norm_rope_3d_tables: q and k rotated in place, pre-RoPE k staged."""
+    _ops.fused_qk_norm_rope_3d_tables_kstage(q, k, k_stage, seq_len, num_heads, eps, q_weight,
+                                             k_weight, cos, sin)
 
 
 def kv_ring_slot(t0: int, frames_per_chunk: int, cache_slots: int) -> int:

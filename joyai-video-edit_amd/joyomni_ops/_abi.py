@@ -58,6 +58,9 @@ SIGNATURES: dict[str, list] = {
     "jo_fused_qk_norm_rope_3d_grid_kstage": [
         _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _F, _P, _P, _P,
         c_int32, c_int32, c_int32, c_int32, c_int32, _F, _P],
+    "jo_fused_qk_norm_rope_3d_tables": [
+        _P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64,
+        _I64, _I64, _F, _P, _P, _P, _P, _I64, c_int32, _P],
     "jo_fused_qk_norm_rope_3d_kvcache": [
         _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64,
         _F, _P, _P, _P, c_int32, c_int32, c_int32, c_int32, c_int32, _F, _P],
