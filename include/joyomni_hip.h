@@ -65,13 +65,12 @@ int jo_abi_version(void);
  *                       4, 6 or 8 (env JO_QK_SPLIT)
  *   JO_KNOB_KV_SPLIT    1 = K and V of a KV-pool row on one wave, 2 = on two
  *                       (env JO_KV_SPLIT)
- *   JO_KNOB_GEMM_SHAPE  FP8 GEMM tile: 0 = 256x256, 1 = 256x128, 2 = the
- *                       register-staged kernel, 3 = 224x256, 4 = 224x128,
- *                       5 = 128x128 and 6 = 64x64 (four waves), 7 = 128x256
- *                       (eight waves), 8 = 64x128, 9 = 128x192 and 10 =
- *                       128x96 (four waves), 11 = 64x96 (two waves; 5-11
- *                       need K % 128 == 0, else the
- *                       register-staged kernel runs) (env JO_GEMM_SHAPE)
+ *   JO_KNOB_GEMM_SHAPE  FP8 GEMM tile: eight waves on 0 = 256x256, 1 = 208x256,
+ *                       3 = 224x256, 4 = 160x256, 7 = 128x256 or 9 = 112x256;
+ *                       5 = 128x128, 6 = 64x64, 8 = 64x128 and 10 = 128x96
+ *                       (four waves), 11 = 64x96 (two waves); 2 = the
+ *                       register-staged kernel, which also runs where 5-11
+ *                       are forced and K % 128 != 0 (env JO_GEMM_SHAPE)
  *   JO_KNOB_GEMM_SPLIT  FP8 GEMM K split: 1 (none), 2, 4 or 8 workgroups per
  *                       tile, taken by the 128x128 and 64x64 tiles when
  *                       jo_fp8_scaled_mm_ws has the workspace for it and

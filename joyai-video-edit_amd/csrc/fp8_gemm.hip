@@ -28,6 +28,7 @@ namespace {
 
 typedef int i32x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kBM = 256;
 constexpr int kBN = 256;
@@ -45,6 +46,7 @@ struct GemmArgs {
   int64_t lda, ldb, ldo;
   int M, N, K;
   float* ws = nullptr;  // split K: fp32 partial products [splits, M, N]
+  int group = 4;        // tile rows of a group (xcd_grouped_tile)
 };
 
 __device__ __forceinline__ int swz(int r) { return (r & 7) ^ ((r >> 3) & 1); }
@@ -53,6 +55,11 @@ __device__ __forceinline__ int swz(int r) { return (r & 7) ^ ((r >> 3) & 1); }
 // v_mfma_f32_32x32x64_f8f6f4).
 __device__ __forceinline__ f32x16 mfma32(const i32x8& a, const i32x8& b, const f32x16& c) {
   return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, c, 0, 0, 0, 0, 0, 0);
+}
+
+// One 16x16x128 fp8 MFMA with unit block scales.
+__device__ __forceinline__ f32x4 mfma16(const i32x8& a, const i32x8& b, const f32x4& c) {
+  return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, c, 0, 0, 0, 0, 0, 0);
 }
 
 template <class OutTag>
@@ -513,27 +520,49 @@ void launch_pipe(const GemmArgs& g, hipStream_t stream) {
 }
 
 // ---------------------------------------------------------------------------
-// 128-byte-stage kernel (K % 128 == 0), the default for 8-wave tiles: the
-// tile and wave layout of the pipelined kernel, but K advances in 128-byte
-// stages through two LDS slots of (BM + BN) x 128 bytes. A wave's 1 KB direct
-// load then covers eight whole 128-byte lines (eight lanes per row) where a
-// 64-byte stage covers sixteen half lines. The loads are what bounds the K
-// loop (a timing-only copy of the 64-byte kernel without them ran 4096^3 in
-// 48 instead of 65 us), and the vector L1 stalls on its pending misses to L2:
-// whole lines halve the L1 -> L2 requests for the same bytes (rocprofv3
-// TCP_TCC_READ_REQ) and took 4096^3 from 67.7 to 61.2 us. Per stage s, one
-// barrier:
-//   MFMAs of the first 64-byte half    | reads of the second half's fragments
+// Pair kernel (K % 128 == 0), the default for many rows: eight waves on a
+// BM x 256 tile (BM a multiple of 16 from 96 to 256), two per SIMD, in a 2 x 4
+// grid of wave tiles of 64 columns whose first row takes (BM / 16 + 1) / 2 of
+// the 16-row blocks. K advances in 128-byte stages, one
+// v_mfma_f32_16x16x128_f8f6f4 deep, through LDS slots that direct
+// global->LDS loads fill (eight lanes a row: a 1 KB load covers eight whole
+// 128-byte lines; half lines doubled the L1 -> L2 requests and cost 10%). Per
+// stage s, one barrier:
+//   MFMAs of the wave's first two column blocks  | reads of the rest of this
+//                                                | stage's fragments
 //   wait for those reads and for this wave's loads of stage s+1; barrier
-//   MFMAs of the second half | loads of stage s+2 into the slot of stage s
-//   (every wave holds its fragments now), reads of stage s+1's first half.
+//   MFMAs of the last two | loads of stage s+2 into the slot of stage s (every
+//                         | wave holds its fragments now), reads of stage
+//                         | s+1's first fragments into registers set free
+// so every fragment register is loaded under MFMAs that do not need it.
 // LDS rows are 128 bytes; chunk c of row r sits at chunk position
 // c ^ ((r >> 1) & 7): the sixteen consecutive rows a 16-lane group reads with
 // one ds_read_b128 then fall in sixteen distinct 16-byte bank groups.
+//
+// What bounds it is power: with random operands the MFMAs alone (from
+// registers, no memory) run at 4.0 PFLOP/s, the clock falling to ~1.95 GHz,
+// and at 3.7 with 32x32x64, whose accumulators move twice the bits per flop. A
+// 208-row stage takes ~2050 cycles for 1664 of MFMAs at 1.85-1.95 GHz, and
+// forms with fewer idle cycles run at lower clocks for the same time (four
+// waves of 128 x 128, with a third less LDS traffic: 2-12% slower). Measured
+// against the same tiles on 32x32x64 with 224 or 256 rows only:
+// 3120x12288x4096 130 -> 123.5 us, 3120x16384x4096 173 -> 162,
+// 3120x4096x16384 168 -> 164, 3120x4096x4096 45 -> 41.5, 4096^3 55 -> 52,
+// 8192^3 408 -> 393 (2.8 PFLOP/s), 1560x12288x4096 80.5 -> 67,
+// 1560x4096x4096 32 -> 26, 512x12288x4096 30.7 -> 26.7.
 // ---------------------------------------------------------------------------
 constexpr int kQBK = 128;  // bytes of K per stage
 
 __device__ __forceinline__ int qswz(int r) { return (r >> 1) & 7; }
+
+// fn(std::integral_constant<int, 0>) .. fn(std::integral_constant<int, N - 1>).
+template <int N, int I = 0, class Fn>
+__device__ __forceinline__ void static_for(Fn&& fn) {
+  if constexpr (I < N) {
+    fn(std::integral_constant<int, I>{});
+    static_for<N, I + 1>(fn);
+  }
+}
 
 // Direct loads of one stage: BM rows of A then BN rows of B^T, 128 bytes
 // each, written by (BM + BN) / 8 wave instructions of 1 KB (8 rows, eight
@@ -549,15 +578,27 @@ struct PairLoads {
   bool last;                      // the wave owns a slot kPerWave - 1 (always when kEven)
 };
 
-// NBS: B stages go through a ring of NBS slots beside A's two, so B loads run
-// NBS - 1 stages ahead and A loads one (NBS = 3 for one-round grids, below).
+// LDS of a workgroup: the rings (later the staged output tile), then the row
+// scales, column scales and bias of the tile.
+constexpr int kScaleRows = 256;
+template <int BM, int BN, int NW, int NBS>
+constexpr int pair_ring_bytes() {
+  constexpr int ring = (2 * BM + NBS * BN) * kQBK;
+  constexpr int store = NW * ((BM / 16 + 1) / 2) * 16 * (BN / (NW / 2) * 2 + 16);
+  return ring > store ? ring : store;
+}
+
+// The K loop and epilogue of a wave holding MI row blocks of 16 (from the
+// tile's row row0 on). NBS: B stages go through a ring of NBS slots beside A's
+// two, so B loads run NBS - 1 stages ahead and A loads one.
 template <class OutTag, int BM, int BN, int NW, int MI, int NBS>
 __device__ __forceinline__ void fp8_gemm_pair_tile(const GemmArgs& g, uint8_t* smem,
                                                    const PairLoads<BM, BN, NW>& ld, int wave,
-                                                   int wm, int wn, int m0, int n0) {
+                                                   int row0, int wn, int m0, int n0) {
   using Loads = PairLoads<BM, BN, NW>;
   constexpr int WCOLS = BN / (NW / 2);  // wave tile columns
-  constexpr int J = WCOLS / 32;         // n-subtiles of 32 per wave
+  constexpr int J = WCOLS / 16;         // n-blocks of 16 per wave
+  constexpr int JH = J / 2;             // n-blocks of a half stage
   // Ring layout. NBS = 2: slot t % 2 holds stage t's A rows then its B rows.
   // NBS = 3: two A slots, then three B slots.
   constexpr int kASlot = NBS == 2 ? (BM + BN) * kQBK : BM * kQBK;
@@ -565,84 +606,70 @@ __device__ __forceinline__ void fp8_gemm_pair_tile(const GemmArgs& g, uint8_t* s
   constexpr int kBBase = NBS == 2 ? BM * kQBK : 2 * BM * kQBK;
   constexpr int PER = Loads::kPerWave;
   constexpr int NB = BN / 8 / NW;  // B loads of a wave a stage: the last NB of its slots
-  static_assert(J >= 1 && MI >= 2 && MI <= 4, "tile shape");
+  static_assert(J >= 2 && J % 2 == 0 && MI >= 2 && MI <= 8, "tile shape");
+  constexpr int kScaleOff = pair_ring_bytes<BM, BN, NW, NBS>();
   static_assert((NBS == 2 || NBS == 3) && (BN / 8) % NW == 0, "B ring");
-  static_assert(128 * (BN * 2 + 16) <= (2 * BM + NBS * BN) * kQBK, "epilogue staging fits the rings");
   const int lane = threadIdx.x % kWave;
   const int stages = g.K / kQBK;
   // Load i of this wave is A (slot index below BM / 8; a wave's A loads come
-  // first in its slot order) or B; stage t of it goes to ring slot t % 2 or
-  // t % NBS.
-  auto is_a = [&](int i) { return wave + i * NW < BM / 8; };
-  auto issue_one = [&](int t, int i) {
+  // first in its slot order) or B: known at compile time but for the one index
+  // that the last A slots share with the first B slots.
+  auto is_a = [&](auto ic) {
+    constexpr int i = decltype(ic)::value;
+    if constexpr ((i + 1) * NW <= BM / 8) return true;
+    if constexpr (i * NW >= BM / 8) return false;
+    return wave + i * NW < BM / 8;
+  };
+  // Load i of stage t, A to slot t % 2 and B to ring slot bslot.
+  auto issue_one = [&](int t, int bslot, auto ic) {
+    constexpr int i = decltype(ic)::value;
     if (Loads::kEven || i + 1 < PER || ld.last) {
-      if constexpr (NBS == 2)
-        __builtin_amdgcn_global_load_lds(ld.base[i] + (ld.off[i] + t * kQBK), (__attribute__((address_space(3))) void*)(smem + (t & 1) * kASlot + (wave + i * NW) * 1024), 16, 0, 0);
-      else
-        __builtin_amdgcn_global_load_lds(ld.base[i] + (ld.off[i] + t * kQBK), (__attribute__((address_space(3))) void*)(is_a(i) ? smem + (t & 1) * kASlot + (wave + i * NW) * 1024 : smem + kBBase + (t % NBS) * kBSlot + (wave + i * NW - BM / 8) * 1024), 16, 0, 0);
+      uint8_t* dst = is_a(ic) || NBS == 2 ? smem + (t & 1) * kASlot + (wave + i * NW) * 1024
+                                          : smem + kBBase + bslot * kBSlot + (wave + i * NW - BM / 8) * 1024;
+      __builtin_amdgcn_global_load_lds(ld.base[i] + (ld.off[i] + t * kQBK), (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
     }
   };
   // The loads issued in stage s's second half: A of stage s + 2 and B of
-  // stage s + NBS.
-  auto issue_batch_one = [&](int s, int i) {
-    if constexpr (NBS == 2)
-      issue_one(s + 2, i);
-    else if (is_a(i))
-      issue_one(s + 2, i);
+  // stage s + NBS, the latter into the slot of stage s's B (bcur).
+  auto issue_batch_one = [&](int s, int bcur, auto ic) {
+    if (NBS == 2 || is_a(ic))
+      issue_one(s + 2, 0, ic);
     else if (s + NBS < stages)
-      issue_one(s + NBS, i);
+      issue_one(s + NBS, bcur, ic);
   };
 
-  f32x16 acc[MI][J];
+  f32x4 acc[MI][J];
 #pragma unroll
   for (int i = 0; i < MI; ++i)
 #pragma unroll
-    for (int j = 0; j < J; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+    for (int j = 0; j < J; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  // Fragment rows are wm*128 + i*32 + lane%32 (A) and wn*WCOLS + j*32 +
-  // lane%32 (B): all differ from lane%32 by multiples of 16, so they share
-  // its swizzle, and row block i (j) sits i*32 (j*32) rows after block 0.
-  const int fr = lane & 31, fh = lane >> 5;
+  // Fragment rows are row0 + i*16 + lane%16 (A) and wn*WCOLS + j*16 +
+  // lane%16 (B): they differ from lane%16 by multiples of 16, so they share
+  // its swizzle. Lane group lane/16 holds the 32 bytes of K from its chunk
+  // pair on, in A and B alike.
+  const int fr = lane & 15, fh = lane >> 4;
   const int q = qswz(fr);
-  int offa[2][2], offb[2][2];  // [half of the stage][chunk of the pair]
+  int offa[2], offb[2];  // [chunk of the pair]
 #pragma unroll
-  for (int k = 0; k < 2; ++k)
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int pos = ((k * 4 + fh * 2 + h) ^ q) << 4;
-      offa[k][h] = (wm * 128 + fr) * kQBK + pos;
-      offb[k][h] = kBBase + (wn * WCOLS + fr) * kQBK + pos;
-    }
-  auto read_frags = [&](int s, int k, i32x8 (&af)[MI], i32x8 (&bf)[J]) {
-    const uint8_t* st = smem + (s & 1) * kASlot;
-    const uint8_t* sb = NBS == 2 ? st : smem + (s % NBS) * kBSlot;
-#pragma unroll
-    for (int j = 0; j < J; ++j) {
-      const u32x4 lo = *reinterpret_cast<const u32x4*>(sb + offb[k][0] + j * 32 * kQBK);
-      const u32x4 hi = *reinterpret_cast<const u32x4*>(sb + offb[k][1] + j * 32 * kQBK);
-      bf[j] = i32x8{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
-    }
-#pragma unroll
-    for (int i = 0; i < MI; ++i) {
-      const u32x4 lo = *reinterpret_cast<const u32x4*>(st + offa[k][0] + i * 32 * kQBK);
-      const u32x4 hi = *reinterpret_cast<const u32x4*>(st + offa[k][1] + i * 32 * kQBK);
-      af[i] = i32x8{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
-    }
+  for (int h = 0; h < 2; ++h) {
+    const int pos = ((fh * 2 + h) ^ q) << 4;
+    offa[h] = (row0 + fr) * kQBK + pos;
+    offb[h] = kBBase + (wn * WCOLS + fr) * kQBK + pos;
+  }
+  auto frag = [&](const uint8_t* lo_p, const uint8_t* hi_p) {
+    const u32x4 lo = *reinterpret_cast<const u32x4*>(lo_p);
+    const u32x4 hi = *reinterpret_cast<const u32x4*>(hi_p);
+    return i32x8{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
   };
-  // Fragment f of half k of stage s: B block f (f < J), else A block f - J.
-  auto read_one = [&](int s, int k, int f, i32x8 (&af)[MI], i32x8 (&bf)[J]) {
-    const uint8_t* st = (NBS == 2 || f >= J) ? smem + (s & 1) * kASlot : smem + (s % NBS) * kBSlot;
-    const int off = f < J ? offb[k][0] + f * 32 * kQBK : offa[k][0] + (f - J) * 32 * kQBK;
-    const int off2 = f < J ? offb[k][1] + f * 32 * kQBK : offa[k][1] + (f - J) * 32 * kQBK;
-    const u32x4 lo = *reinterpret_cast<const u32x4*>(st + off);
-    const u32x4 hi = *reinterpret_cast<const u32x4*>(st + off2);
-    const i32x8 v{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
-    if (f < J)
-      bf[f] = v;
-    else
-      af[f - J] = v;
+  i32x8 af[MI], bf[J];
+  auto read_a = [&](int s, int i) {
+    const uint8_t* st = smem + (s & 1) * kASlot;
+    af[i] = frag(st + offa[0] + i * 16 * kQBK, st + offa[1] + i * 16 * kQBK);
+  };
+  auto read_b = [&](int bslot, int j) {
+    const uint8_t* st = smem + bslot * kBSlot;
+    bf[j] = frag(st + offb[0] + j * 16 * kQBK, st + offb[1] + j * 16 * kQBK);
   };
   // Stage s's wait: this wave's LDS reads, and its loads up to stage s + 1's.
   // A of s + 1 came with the latest loads; with NBS = 3 only their tail, B of
@@ -660,64 +687,58 @@ __device__ __forceinline__ void fp8_gemm_pair_tile(const GemmArgs& g, uint8_t* s
     asm volatile("" ::: "memory");
   };
   // B first: the accumulator is the transposed tile (a lane holds one output
-  // row and, per group of four registers, four consecutive columns).
-  auto mfma_q = [&](int qi, i32x8 (&af)[MI], i32x8 (&bf)[J]) {
-    acc[qi / J][qi % J] = mfma32(bf[qi % J], af[qi / J], acc[qi / J][qi % J]);
+  // row and four consecutive columns). MFMA t of a half: row block t / JH,
+  // column block half * JH + t % JH.
+  auto mfma_t = [&](int half, int t) {
+    const int i = t / JH, j = half * JH + ((i & 1) ? JH - 1 - t % JH : t % JH);
+    acc[i][j] = mfma16(bf[j], af[i], acc[i][j]);
   };
-
-  i32x8 a0[MI], b0[J], a1[MI], b1[J];  // fragments of the first / second half of a stage
-  // With 256-row tiles the first KB MFMAs of the second half go out before
-  // the barrier (their fragments are this wave's own), so the matrix cores
-  // are busy while the waves meet.
-  constexpr int KB = BM == 256 ? 2 : 0;
-  // Stage s with stage s+1 present (NEXT) and stage s+2 present (MORE).
-  auto stage = [&](int s, auto next, auto more) {
+  constexpr int NT = MI * JH;     // MFMAs of a half
+  constexpr int NA1 = MI / 2;     // A blocks read in the first half (the last ones)
+  constexpr int NA0 = MI - NA1;   // A blocks read in the second half, for the next stage
+  // Fragment f that the first half reads (of this stage), in the order of
+  // need: A blocks NA0 .. MI-1, then the second half's B blocks.
+  auto read_first = [&](int s, int bcur, int f) {
+    if (f < NA1)
+      read_a(s, NA0 + f);
+    else
+      read_b(bcur, JH + f - NA1);
+  };
+  constexpr int NF1 = NA1 + JH;
+  // Stage s with stage s+1 present (NEXT) and stage s+2 present (MORE); bcur
+  // and bnext are the ring slots of stage s's and stage s+1's B.
+  constexpr int KB = BM == 256 ? 2 : 0;  // MFMAs of the second half before the barrier
+  auto stage = [&](int s, int bcur, int bnext, auto next, auto more) {
     constexpr bool kNext = decltype(next)::value, kMore = decltype(more)::value;
-    // First half: MFMAs on a0/b0 while the second half's fragments arrive.
-    read_frags(s, 1, a1, b1);
 #pragma unroll
-    for (int qi = 0; qi < MI * J; ++qi) mfma_q(qi, a0, b0);
-#pragma unroll
-    for (int qi = 0; qi < MI * J; ++qi) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
-      __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);  // DS read
+    for (int t = 0; t < NT; ++t) {
+      mfma_t(0, t);
+      if (t < NF1) read_first(s, bcur, t);
+      __builtin_amdgcn_sched_barrier(0);
     }
+#pragma unroll
+    for (int f = NT; f < NF1; ++f) read_first(s, bcur, f);
     __builtin_amdgcn_sched_barrier(0);
     wait_next(s);
 #pragma unroll
-    for (int qi = 0; qi < KB; ++qi) mfma_q(qi, a1, b1);
+    for (int t = 0; t < KB; ++t) mfma_t(1, t);
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (kNext) bare_barrier();
-    // Second half, in a fixed order: each MFMA followed by up to two of stage
-    // s+2's loads (the first four MFMAs carry them) and one of stage s+1's
-    // first-half fragments. Issuing all of the stage's loads at once after the
-    // barrier measured 2-4% slower on 4096^3 and the 3120-row qkv / MLP-up
-    // shapes (level on the one-round MLP-down and attention-out shapes).
-    constexpr int NQ = MI * J - KB;  // MFMAs after the barrier
-    constexpr int NF = J + MI;       // fragments of the next first half
-#pragma unroll
-    for (int t = 0; t < NQ; ++t) {
-      mfma_q(KB + t, a1, b1);
-      if constexpr (kMore) {
-#pragma unroll
-        for (int u = 0; u < 2; ++u)
-          if (2 * t + u < PER) issue_batch_one(s, 2 * t + u);
-      }
+    static_for<NT - KB>([&](auto uc) {
+      constexpr int u = decltype(uc)::value, t = KB + u;
+      mfma_t(1, t);
+      if constexpr (kMore && u < PER) issue_batch_one(s, bcur, uc);
       if constexpr (kNext) {
-        if (t < NF) read_one(s + 1, 0, t, a0, b0);
+        // B blocks of the next first half, then A block i once its own MFMAs
+        // of this half are out.
+        if constexpr (u < JH) read_b(bnext, u);
+        if constexpr (t % JH == JH - 1 && t / JH >= 1 && t / JH - 1 < NA0) read_a(s + 1, t / JH - 1);
       }
       __builtin_amdgcn_sched_barrier(0);
-    }
-    if constexpr (kNext) {
-#pragma unroll
-      for (int f = NQ; f < NF; ++f) read_one(s + 1, 0, f, a0, b0);
-    }
-    if constexpr (kMore) {
-#pragma unroll
-      for (int i = 2 * NQ; i < PER; ++i) issue_batch_one(s, i);
-    }
-    __builtin_amdgcn_sched_barrier(0);
+    });
+    static_assert(PER <= NT - KB, "every load has an MFMA to follow");
   };
+  static_assert(NA0 <= MI - 1 && NT - KB >= JH, "the second half reads every early fragment");
 
   using T = std::true_type;
   using F = std::false_type;
@@ -725,29 +746,39 @@ __device__ __forceinline__ void fp8_gemm_pair_tile(const GemmArgs& g, uint8_t* s
   // have issued (stage 1; with NBS = 3, A of 1 and B of 1 and 2, B before A
   // within a stage); stage 0 starts once its own loads are in.
   auto issue_part = [&](int t, bool a) {
-#pragma unroll
-    for (int i = 0; i < PER; ++i)
-      if (is_a(i) == a) issue_one(t, i);
+    static_for<PER>([&](auto ic) {
+      if (is_a(ic) == a) issue_one(t, t, ic);
+    });
   };
+  auto issue = [&](int t) { static_for<PER>([&](auto ic) { issue_one(t, t, ic); }); };
+  // The tile's scales and bias go to LDS first (4 bytes a lane, 64 lanes a
+  // load), the oldest loads of all, so that the epilogue does not start with
+  // a wait for memory.
+  uint8_t* scales = smem + kScaleOff;
+  {
+    auto load4 = [&](const void* src, int at) {
+      __builtin_amdgcn_global_load_lds(static_cast<const uint8_t*>(src), (__attribute__((address_space(3))) void*)(scales + at), 4, 0, 0);
+    };
+    static_assert(BN == 256 && NW == 8 && kScaleRows == 256, "one scale load a wave");
+    if (wave < 4)
+      load4(g.sa + min(m0 + wave * 64 + lane, g.M - 1), wave * 256);
+    else
+      load4(g.sb + min(n0 + (wave - 4) * 64 + lane, g.N - 1), wave * 256);
+    if (g.bias && wave < 2)
+      load4(static_cast<const uint16_t*>(g.bias) + min(n0 + (wave * 64 + lane) * 2, g.N - 2), 2048 + wave * 256);
+  }
   // In flight after stage 0's loads: NB B loads per later B stage and this
   // wave's A loads of stage 1 (PER - NB; one fewer for a wave without a last
   // slot, which is always a B slot since every wave has NB of those).
   const bool full = Loads::kEven || ld.last;
   if constexpr (NBS == 2) {
-    auto issue = [&](int t) {
-#pragma unroll
-      for (int i = 0; i < PER; ++i) issue_one(t, i);
-    };
-    auto wait_own = [&](int later) {
-      JO_WAIT_LDS0();
-      if (Loads::kEven || ld.last)
-        wait_loads<PER>(later);
-      else
-        wait_loads<PER - 1>(later);
-    };
     issue(0);
     if (stages > 1) issue(1);
-    wait_own(stages > 1 ? 1 : 0);
+    JO_WAIT_LDS0();
+    if (full)
+      wait_loads<PER>(stages > 1 ? 1 : 0);
+    else
+      wait_loads<PER - 1>(stages > 1 ? 1 : 0);
   } else {
     issue_part(0, false);
     issue_part(0, true);
@@ -761,8 +792,7 @@ __device__ __forceinline__ void fp8_gemm_pair_tile(const GemmArgs& g, uint8_t* s
       else
         JO_WAIT_VM(2 * NB + PER - NB - 1);
     } else if (stages == 2) {
-#pragma unroll
-      for (int i = 0; i < PER; ++i) issue_one(1, i);
+      issue(1);
       JO_WAIT_LDS0();
       if (full)
         JO_WAIT_VM(PER);
@@ -774,34 +804,103 @@ __device__ __forceinline__ void fp8_gemm_pair_tile(const GemmArgs& g, uint8_t* s
     }
   }
   bare_barrier();
-  read_frags(0, 0, a0, b0);
-  int s = 0;
-  for (; s + 2 < stages; ++s) stage(s, T{}, T{});
-  if (s + 1 < stages) stage(s++, T{}, F{});
-  stage(s, F{}, F{});
+#pragma unroll
+  for (int j = 0; j < JH; ++j) read_b(0, j);  // stage 0's slot
+#pragma unroll
+  for (int i = 0; i < NA0; ++i) read_a(0, i);
+  int s = 0, bcur = 0, bnext = 1, bthen = NBS - 1;  // bthen: NBS = 3 only
+  auto turn = [&]() {
+    const int freed = bcur;
+    bcur = bnext;
+    bnext = NBS == 2 ? freed : bthen;
+    bthen = freed;
+  };
+  for (; s + 2 < stages; ++s, turn()) stage(s, bcur, bnext, T{}, T{});
+  if (s + 1 < stages) {
+    stage(s++, bcur, bnext, T{}, F{});
+    turn();
+  }
+  stage(s, bcur, bnext, F{}, F{});
 
-  store_tile<OutTag, BM, BN, NW, MI>(g, smem, acc, wm, wn, m0, n0);
+  // Epilogue. Block (i, j) element e of a lane is row m0 + row0 + i*16 +
+  // lane%16, column n0 + wn*WCOLS + j*16 + (lane/16)*4 + e. Each wave passes
+  // its tile through its own part of the LDS (the ring is free once every
+  // wave is past the barrier), one block of 16 rows at a time, so that rows
+  // leave as whole 16-byte lane stores, WCOLS * 2 bytes (128: a whole line) a
+  // row. No wave waits for another after the barrier.
+  constexpr int kRowBytes = WCOLS * 2 + 16;
+  constexpr int kWaveBytes = MI * 16 * kRowBytes;
+  float sam[MI];
+#pragma unroll
+  for (int i = 0; i < MI; ++i) sam[i] = *reinterpret_cast<const float*>(scales + (row0 + i * 16 + fr) * 4);
+  float sbq[J][4], bq[J][4];
+#pragma unroll
+  for (int j = 0; j < J; ++j) {
+    const int c = wn * WCOLS + j * 16 + fh * 4;
+    const u32x4 sbv = *reinterpret_cast<const u32x4*>(scales + kScaleRows * 4 + c * 4);
+    const u32x2 braw = *reinterpret_cast<const u32x2*>(scales + kScaleRows * 4 + BN * 4 + c * 2);
+    const u32x4 b4{braw.x, braw.y, 0u, 0u};
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      sbq[j][t] = elem<F32>(sbv, t);
+      bq[j][t] = g.bias ? elem<OutTag>(b4, t) : 0.f;
+    }
+  }
+  bare_barrier();  // this wave's LDS reads were all waited for by its last MFMAs
+  constexpr int kMaxWave = ((BM / 16 + 1) / 2) * 16 * kRowBytes;
+  static_assert(kWaveBytes <= kMaxWave, "wave region");
+  uint8_t* mine = smem + wave * kMaxWave;
+  constexpr int kLanesPerRow = WCOLS * 2 / 16;          // 16-byte lanes of a row
+  constexpr int kRowsPerStore = kWave / kLanesPerRow;   // rows of a wave store
+  const int sr = lane / kLanesPerRow, sc = lane % kLanesPerRow;
+  auto stage_block = [&](int i) {
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      float o[8];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        o[t] = __builtin_fmaf(sam[i], acc[i][j][t] * sbq[j][t], bq[j][t]);
+        o[t + 4] = 0.f;
+      }
+      const u32x4 pk = pack<OutTag>(o);
+      *reinterpret_cast<u32x2*>(mine + (i * 16 + fr) * kRowBytes + (j * 16 + fh * 4) * 2) = u32x2{pk.x, pk.y};
+    }
+  };
+  // A wave's LDS operations run in order, so block i's reads follow its
+  // writes; block i + 1 is written before block i leaves.
+  stage_block(0);
+#pragma unroll
+  for (int i = 0; i < MI; ++i) {
+    if (i + 1 < MI) stage_block(i + 1);
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int r = i * 16; r < i * 16 + 16; r += kRowsPerStore) {
+      const int m = m0 + row0 + r + sr, n = n0 + wn * WCOLS + sc * 8;
+      const u32x4 v = *reinterpret_cast<const u32x4*>(mine + (r + sr) * kRowBytes + sc * 16);
+      if (m < g.M && n < g.N)
+        st16_nt(static_cast<uint16_t*>(g.out) + static_cast<int64_t>(m) * g.ldo + n, v);
+    }
+  }
 }
 
 // Output tile of this workgroup. The dispatcher hands workgroup id (linear
 // over the grid, x fastest) to XCD id % 8, and each XCD has its own L2, so
 // consecutive ids are spread over the XCDs and the tiles an XCD runs
 // together should share operand rows. XCD x gets a contiguous range of a
-// grouped order (groups of four tile rows, column by column inside a group):
-// the ~32 tiles it runs at once are four tile rows by eight columns, twelve
-// operand panels where the row-major order gives it two columns by sixteen
-// rows, eighteen (3120x12288x4096 141.0 -> 137.5 us, 3120x4096x16384
-// 180.6 -> 176.3 us, 4096^3 59.0 -> 58.1 us).
-__device__ __forceinline__ void xcd_grouped_tile(int bm, int bn, int& m0, int& n0) {
-  constexpr int kGroup = 4;
+// grouped order (groups of `group` tile rows, column by column inside a
+// group): the ~32 tiles it runs at once are five tile rows by six columns,
+// eleven operand panels where the row-major order gives it two columns by
+// sixteen rows, eighteen (3120x12288x4096 141.0 -> 137.5 us with groups of
+// four, 4096^3 59.0 -> 58.1). group_rows picks the size.
+__device__ __forceinline__ void xcd_grouped_tile(int group, int bm, int bn, int& m0, int& n0) {
   const int ntn = gridDim.x, ntm = gridDim.y, tiles = ntn * ntm;
   const int id = blockIdx.y * ntn + blockIdx.x;
   const int x = id & 7;
   const int t = x * (tiles >> 3) + min(x, tiles & 7) + (id >> 3);  // a bijection of [0, tiles)
-  const int grp = t / (kGroup * ntn);
-  const int r0 = grp * kGroup;
-  const int rows = min(kGroup, ntm - r0);
-  const int w = t - grp * kGroup * ntn;
+  const int grp = t / (group * ntn);
+  const int r0 = grp * group;
+  const int rows = min(group, ntm - r0);
+  const int w = t - grp * group * ntn;
   m0 = (r0 + w % rows) * bm;
   n0 = (w / rows) * bn;
 }
@@ -809,16 +908,18 @@ __device__ __forceinline__ void xcd_grouped_tile(int bm, int bn, int& m0, int& n
 template <class OutTag, int BM, int BN, int NW, int NBS>
 __device__ __forceinline__ void fp8_gemm_pair_body(const GemmArgs& g) {
   using Loads = PairLoads<BM, BN, NW>;
-  static_assert(BM == 256 || BM == 224, "tile rows");
-  __shared__ __attribute__((aligned(1024))) uint8_t smem[(2 * BM + NBS * BN) * kQBK];
+  constexpr int RB = BM / 16;  // 16-row blocks: the first wave row takes (RB + 1) / 2
+  static_assert(BM % 16 == 0 && BM >= 64 && BM <= 256, "tile rows");
+  __shared__ __attribute__((aligned(1024))) uint8_t smem[pair_ring_bytes<BM, BN, NW, NBS>() + (kScaleRows + BN) * 4 + BN * 2];
   const int tid = threadIdx.x;
   const int lane = tid % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
-  // Wave tiles as in fp8_gemm_pipe_body.
-  const int wm = BM == 256 ? (wave & 1) : wave / (NW / 2);
-  const int wn = BM == 256 ? (wave >> 1) : wave % (NW / 2);
+  // A 2 x NW/2 grid of wave tiles. A workgroup's waves are spread round-robin
+  // over the CU's four SIMDs, so with NW = 8 waves w and w + 4 share a SIMD:
+  // with an odd number of row blocks each SIMD runs a wave of each height.
+  const int wm = wave / (NW / 2), wn = wave % (NW / 2);
   int m0, n0;
-  xcd_grouped_tile(BM, BN, m0, n0);
+  xcd_grouped_tile(g.group, BM, BN, m0, n0);
 
   // Lane p of a slot fills row +p/8, chunk position p%8 with the global chunk
   // that belongs there. Rows beyond M (N) read row M-1 (N-1); they are never
@@ -836,25 +937,55 @@ __device__ __forceinline__ void fp8_gemm_pair_body(const GemmArgs& g) {
                 (((lane & 7) ^ qswz(r)) * 16);
   }
   ld.last = Loads::kEven || wave + (Loads::kPerWave - 1) * NW < Loads::kSlots;
-  if constexpr (BM == 256) {
-    fp8_gemm_pair_tile<OutTag, BM, BN, NW, 4, NBS>(g, smem, ld, wave, wm, wn, m0, n0);
+  constexpr int kUp = (RB + 1) / 2, kLow = RB / 2;
+  if constexpr (kUp == kLow) {
+    fp8_gemm_pair_tile<OutTag, BM, BN, NW, kUp, NBS>(g, smem, ld, wave, wm * kUp * 16, wn, m0, n0);
   } else {
     if (wm == 0)
-      fp8_gemm_pair_tile<OutTag, BM, BN, NW, 4, NBS>(g, smem, ld, wave, wm, wn, m0, n0);
+      fp8_gemm_pair_tile<OutTag, BM, BN, NW, kUp, NBS>(g, smem, ld, wave, 0, wn, m0, n0);
     else
-      fp8_gemm_pair_tile<OutTag, BM, BN, NW, 3, NBS>(g, smem, ld, wave, wm, wn, m0, n0);
+      fp8_gemm_pair_tile<OutTag, BM, BN, NW, kLow, NBS>(g, smem, ld, wave, kUp * 16, wn, m0, n0);
   }
 }
 
 template <class OutTag, int BM, int BN, int NW, int NBS>
-__global__ __launch_bounds__(NW * 64, 8 / NW) void fp8_gemm_pair_kernel(const GemmArgs g) {
+__global__ __launch_bounds__(NW * 64, 1) void fp8_gemm_pair_kernel(const GemmArgs g) {
   fp8_gemm_pair_body<OutTag, BM, BN, NW, NBS>(g);
 }
 
-template <class OutTag, int BM, int BN, int NW, int NBS = 2>
-void launch_pair(const GemmArgs& g, hipStream_t stream) {
+// Tile rows of a group of xcd_grouped_tile: equal groups of at most five (six
+// rows stay one group). Against four: [3120, 12288] x 4096 at fifteen tile
+// rows 123.3 -> 121.5 us (three groups of five against 4 + 4 + 4 + 3),
+// [512, 12288] x 4096 at five tile rows 28.8 -> 26.7 (one group: the weight
+// leaves HBM once); two, three, eight and one group of all rows measured level
+// or slower on eleven shapes.
+int group_rows(int tile_rows) {
+  if (tile_rows <= 6) return tile_rows;
+  const int groups = (tile_rows + 4) / 5;
+  return (tile_rows + groups - 1) / groups;
+}
+
+template <class OutTag, int BM, int BN, int NW, int NBS>
+void launch_pair(const GemmArgs& args, hipStream_t stream) {
+  GemmArgs g = args;
+  g.group = group_rows((g.M + BM - 1) / BM);
   hipLaunchKernelGGL((fp8_gemm_pair_kernel<OutTag, BM, BN, NW, NBS>),
                      dim3((g.N + BN - 1) / BN, (g.M + BM - 1) / BM), dim3(NW * 64), 0, stream, g);
+}
+
+// The pair kernel at `rows` tile rows (a multiple of 16 from 96 to 256), B two
+// stages ahead (NBS = 3) except at 256 rows, whose rings fill the LDS: a long
+// K's operands come from HBM and the deeper ring covers their latency
+// ([3120, 4096] x 16384 at 224 rows 174 -> 169 us, [1560, 4096] x 16384 at 192
+// rows 146 -> 123), as it does the loads of the low tiles ([512, 12288] x 4096
+// at 128 rows 28.3 -> 25.7); on multi-round grids of 208 and 224 rows it
+// measured 0-1% slower (169.5 -> 171.0, 168.3 -> 170.8 at 3120x16384x4096).
+template <class OutTag, int ROWS = 256>
+void launch_pair_rows(const GemmArgs& g, hipStream_t stream, int rows) {
+  if (rows == ROWS || ROWS == 96)
+    launch_pair<OutTag, ROWS, 256, 8, (ROWS == 256 ? 2 : 3)>(g, stream);
+  else if constexpr (ROWS > 96)
+    launch_pair_rows<OutTag, ROWS - 16>(g, stream, rows);
 }
 
 // ---------------------------------------------------------------------------
@@ -897,7 +1028,7 @@ __device__ __forceinline__ void fp8_gemm_small_body(const GemmArgs& g) {
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int wm = wave % WGM, wn = wave / WGM;
   int m0, n0;
-  xcd_grouped_tile(BM, BN, m0, n0);
+  xcd_grouped_tile(g.group, BM, BN, m0, n0);
 
   // Lane p of load slot L fills row 8L + p/8 of the stage (A rows, then B^T
   // rows), chunk position p%8, with the global chunk that belongs there; rows
@@ -1109,7 +1240,9 @@ __global__ __launch_bounds__(kBlock) void fp8_gemm_splitk_reduce(const GemmArgs 
 }
 
 template <class OutTag, int BM, int BN, int NW, int NST, int WGM = 2>
-void launch_small(const GemmArgs& g, hipStream_t stream, int splits = 1) {
+void launch_small(const GemmArgs& args, hipStream_t stream, int splits = 1) {
+  GemmArgs g = args;
+  g.group = group_rows((g.M + BM - 1) / BM);
   const dim3 grid((g.N + BN - 1) / BN, (g.M + BM - 1) / BM, splits);
   if (splits == 1) {
     hipLaunchKernelGGL((fp8_gemm_small_kernel<OutTag, BM, BN, NW, NST, false, WGM>), grid,
@@ -1137,59 +1270,71 @@ int cu_count() {
   return n;
 }
 
-// One workgroup per CU at most (a single round of tiles). There the 224-row
-// pair kernel runs its B loads two stages ahead (NBS = 3): with no second
-// round to overlap, the lines wait longer (~530 cycles against ~360 on the
-// multi-round shapes), and the extra stage of B lookahead measured
-// 3120x4096x16384 178 -> 168 us and 3120x4096x4096 50.6 -> 48.1 us (three
-// alternating runs, results bit-identical); on the multi-round shapes and
-// the 256-row tiles (4096^3) it was 3-4% slower.
-bool one_round(const GemmArgs& g, int bm, int bn) {
-  const int64_t tiles = static_cast<int64_t>((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn);
-  return tiles <= cu_count();
+// Launch shapes. kPair + rows: the eight-wave pair kernel with tiles of that
+// many rows x 256 columns (a multiple of 16 from 96 to 256); 2: the
+// register-staged kernel; 5, 6, 8, 10, 11: the small-tile kernel.
+constexpr int kPair = 1000;
+
+// Cost of a pair-kernel launch and of a small-tile one in the same unit, a
+// small-tile kernel's operand bytes per K byte on the busiest CU (those run at
+// about 49 KB/us a CU). The pair kernel's stage takes about 9.6 rows + 80
+// cycles (measured 2450 at 256 rows, 2075 at 208, 1560 at 160, 1325 at 128: the
+// MFMAs), a fifth of that in the unit above at ~2.1 GHz; low tiles are priced
+// higher, by the 32 KB of B a stage that they wait on when the weight comes
+// from HBM ([256, 16384] x 4096 in a whole MLP: 96-row tiles 4 us slower than
+// the 128x128 ones, though level with cached weights).
+int64_t pair_cost(int cus, int M, int N, int rows) {
+  const int64_t tiles = static_cast<int64_t>((M + rows - 1) / rows) * ((N + 255) / 256);
+  const int64_t stage = 96 * rows + 800 > 56 * rows + 8500 ? 96 * rows + 800 : 56 * rows + 8500;
+  return (tiles + cus - 1) / cus * stage / 50;
 }
 
-// Tile rows for the 8-wave x 256-column kernel: one workgroup per CU, so the
-// time is about (rounds of workgroups over the CUs) x (row blocks per SIMD),
-// 8 for a 256-row tile and 7 for a 224-row one. At M = 3120 (13 tiles of 256,
-// 14 of 224) every deployment shape needs the same number of rounds with
-// either height, and 224-row tiles measured 3120x12288x4096 185 -> 180 us,
-// 3120x16384x4096 233 -> 224 us, 3120x4096x16384 198 -> 193 us.
+int64_t small_cost(int cus, int M, int N, int bm, int bn) {
+  const int64_t tiles = static_cast<int64_t>((M + bm - 1) / bm) * ((N + bn - 1) / bn);
+  return (tiles + cus - 1) / cus * (bm + bn);
+}
+
+// The default launch shape, the cheapest of: the pair kernel at every tile
+// height (one workgroup per CU, so what counts is rounds of workgroups times
+// the height, and a height that divides M into whole rounds wastes least: 3120
+// rows are fifteen 208-row tiles, 240 workgroups for 256 CUs at N = 4096), and
+// the small-tile kernel at 128x128, 128x96, 64x128, 64x96 or 64x64 where the
+// 256-column tiles leave CUs idle (ties go to the smaller tile: two 64x64
+// workgroups share a CU). The 96-column tiles cut N = 12288 into 128 columns
+// of tiles, so 128 or 256 rows fill the 256 CUs. Measured on MI355X against
+// the choice of 224- or 256-row tiles (32x32x64 MFMAs) and 128x192 / 128x256
+// small tiles: [3120, 4096] x 4096 45.0 -> 42.7 us (208 rows), [1560, 12288] x
+// 4096 78.4 -> 69.1 (160), [1560, 4096] x 4096 32.2 -> 25.9 (112), [1560, 4096]
+// x 16384 118 -> 101 (112), [512, 12288] x 4096 30.6 -> 25.7 (128); the
+// small tiles at M = 256: [256, 4096] x 4096 34.2 -> 11.4 us (64x64),
+// [256, 12288] x 4096 42.4 -> 22.0 us (128x96).
+int auto_shape(int cus, int M, int N) {
+  int shape = 0;
+  int64_t best = INT64_MAX;
+  for (int rows = 256; rows >= 96; rows -= 16) {
+    const int64_t c = pair_cost(cus, M, N, rows);
+    if (c < best) {
+      best = c;
+      shape = kPair + rows;
+    }
+  }
+  // Larger tiles first: a tie goes to the smaller one.
+  const int small[5][3] = {{5, 128, 128}, {10, 128, 96}, {8, 64, 128}, {11, 64, 96}, {6, 64, 64}};
+  for (const auto& t : small) {
+    const int64_t c = small_cost(cus, M, N, t[1], t[2]);
+    if (c <= best) {
+      best = c;
+      shape = t[0];
+    }
+  }
+  return shape;
+}
+
+// Pair tile rows where K is not whole 128-byte stages (the 64-byte-stage kernel).
 int pick_tile_rows(int M, int N) {
   const int64_t cus = cu_count(), cols = (N + 255) / 256;
   auto cost = [&](int64_t bm) { return ((M + bm - 1) / bm * cols + cus - 1) / cus * (bm / 32); };
   return cost(224) < cost(256) ? 224 : 256;
-}
-
-// The default launch shape. The K loops are bound by the operand bytes each
-// CU streams from L2 (~45 KB/us per CU for every kernel here), so the cost of
-// a shape is (tiles per CU, rounded up) x (BM + BN) bytes per K byte: the 8-wave
-// 224x256 or 256x256 tiles (pick_tile_rows) unless the small-tile kernel at
-// 128x256, 128x192, 128x128, 128x96, 64x128, 64x96 or 64x64 streams fewer bytes on the
-// busiest CU, as where the large tiles leave most CUs idle (ties go to the
-// smaller tile: two 64x64 workgroups share a CU). The 96-column tiles cut
-// N = 12288 into 128 columns of tiles, so 128 or 256 rows fill the 256 CUs.
-// Measured on MI355X, M = 256: [256, 4096] x 4096 34.2 -> 11.4 us (64x64),
-// [256, 12288] x 4096 42.4 -> 24.3 us (128x128) -> 22.0 us (128x96); M = 128,
-// [128, 12288] x 4096 20.4 us (64x128) -> 17.9 us (64x96); M = 1024,
-// [1024, 4096] x 16384 155.4 -> 86.4 us (128x128).
-int auto_shape(int M, int N) {
-  const int64_t cus = cu_count();
-  auto cost = [&](int64_t bm, int64_t bn) {
-    return ((M + bm - 1) / bm * ((N + bn - 1) / bn) + cus - 1) / cus * (bm + bn);
-  };
-  const int bm = pick_tile_rows(M, N);
-  int shape = bm == 224 ? 3 : 0;
-  int64_t best = cost(bm, 256);
-  // Larger tiles first: a tie goes to the smaller one.
-  const int small[7][3] = {{7, 128, 256}, {9, 128, 192}, {5, 128, 128}, {10, 128, 96},
-                            {8, 64, 128}, {11, 64, 96}, {6, 64, 64}};
-  for (const auto& t : small)
-    if (cost(t[1], t[2]) <= best) {
-      best = cost(t[1], t[2]);
-      shape = t[0];
-    }
-  return shape;
 }
 
 // Split K, for few tiles and a long K (the text stream's MLP down: [256,
@@ -1211,37 +1356,39 @@ struct GemmPlan {
   int splits;
 };
 
-void shape_dims(int shape, int M, int N, int& bm, int& bn) {
-  switch (shape) {
-    case 5: bm = 128; bn = 128; break;
-    case 6: bm = 64; bn = 64; break;
-    case 7: bm = 128; bn = 256; break;
-    case 8: bm = 64; bn = 128; break;
-    case 9: bm = 128; bn = 192; break;
-    case 10: bm = 128; bn = 96; break;
-    case 11: bm = 64; bn = 96; break;
-    default: bm = shape == 3 ? 224 : 256; bn = 256; break;
-  }
-  (void)M;
-  (void)N;
-}
-
 int64_t split_bytes(int M, int N, int splits) {
   return splits > 1 ? static_cast<int64_t>(splits) * M * N * 4 : 0;
 }
 
-int64_t plan_cost(int M, int N, int K, int bm, int bn, int splits) {
-  const int64_t cus = cu_count();
+int64_t shape_cost(int cus, int shape, int M, int N) {
+  switch (shape) {
+    case 5: return small_cost(cus, M, N, 128, 128);
+    case 6: return small_cost(cus, M, N, 64, 64);
+    case 8: return small_cost(cus, M, N, 64, 128);
+    case 10: return small_cost(cus, M, N, 128, 96);
+    case 11: return small_cost(cus, M, N, 64, 96);
+    default: return pair_cost(cus, M, N, shape - kPair);
+  }
+}
+
+// Cost of `splits` workgroups sharing each bm x bn small tile's K.
+int64_t split_cost(int cus, int M, int N, int K, int bm, int bn, int splits) {
   const int64_t tiles = static_cast<int64_t>((M + bm - 1) / bm) * ((N + bn - 1) / bn);
-  int64_t c = (tiles * splits + cus - 1) / cus * (bm + bn) * (K / splits);
-  if (splits > 1) c += split_bytes(M, N, splits) / cus + 405 * 1024;
-  return c;
+  return (tiles * splits + cus - 1) / cus * (bm + bn) * (K / splits) + split_bytes(M, N, splits) / cus +
+         405 * 1024;
+}
+
+// The launch shape that a JO_KNOB_GEMM_SHAPE value forces.
+int knob_shape(int v) {
+  constexpr int kShape[12] = {kPair + 256, kPair + 208, 2, kPair + 224, kPair + 160, 5, 6, kPair + 128, 8, kPair + 112, 10, 11};
+  return kShape[v];
 }
 
 GemmPlan plan_gemm(const GemmArgs& g, int64_t ws_bytes) {
   const int forced = launch_knob(JO_KNOB_GEMM_SHAPE);
   const int fsplit = launch_knob(JO_KNOB_GEMM_SPLIT);
-  GemmPlan p{forced >= 0 ? forced : auto_shape(g.M, g.N), 1};
+  const int cus = cu_count();
+  GemmPlan p{forced >= 0 ? knob_shape(forced) : auto_shape(cus, g.M, g.N), 1};
   const int64_t room = ws_bytes < kSplitCap ? ws_bytes : kSplitCap;
   auto split_ok = [&](int sp) {
     return g.K > 0 && g.K % (kQBK * sp) == 0 && split_bytes(g.M, g.N, sp) <= room;
@@ -1251,16 +1398,14 @@ GemmPlan plan_gemm(const GemmArgs& g, int64_t ws_bytes) {
     return p;
   }
   if (forced >= 0) return p;
-  int bm, bn;
-  shape_dims(p.shape, g.M, g.N, bm, bn);
-  const int64_t unsplit = plan_cost(g.M, g.N, g.K, bm, bn, 1);
+  const int64_t unsplit = shape_cost(cus, p.shape, g.M, g.N) * g.K;
   int64_t best = -1;
   GemmPlan split{p.shape, 1};
   const int cand[2][3] = {{5, 128, 128}, {6, 64, 64}};
   for (const auto& c : cand)
     for (int sp = 2; sp <= 8; sp *= 2)
       if (split_ok(sp)) {
-        const int64_t cost = plan_cost(g.M, g.N, g.K, c[1], c[2], sp);
+        const int64_t cost = split_cost(cus, g.M, g.N, g.K, c[1], c[2], sp);
         if (best < 0 || cost < best) {
           best = cost;
           split = GemmPlan{c[0], sp};
@@ -1276,45 +1421,27 @@ int launch_gemm(const GemmArgs& g, hipStream_t stream, int64_t ws_bytes) {
   // when K is 0 and stores the epilogue of a zero accumulator (the bias).
   const bool pipe_ok = g.K > 0 && g.K % kPBK == 0 && aligned(g.sb, 16) && (g.bias == nullptr || aligned(g.bias, 8)) &&
                        256 * (g.lda > g.ldb ? g.lda : g.ldb) + g.K <= int64_t{UINT32_MAX};
-  // 8-wave 256-column tiles measured faster than two 4-wave 128-column
-  // workgroups per CU at every deployment shape (3120x12288x4096: 199 -> 185
-  // us, 3120x16384x4096: 257 -> 233 us). The JO_KNOB_GEMM_SHAPE override
-  // 0|1|2|3|4|5|6|7|8|9|10|11 forces 256x256, 256x128, the register-staged
-  // kernel, 224x256, 224x128, or the small-tile kernel at 128x128, 64x64,
-  // 128x256, 64x128, 128x192, 128x96 or 64x96
-  // (results are the same up to the fp32 accumulation order inside the
-  // matrix cores).
+  // The JO_KNOB_GEMM_SHAPE override forces a shape (knob_shape; results are the
+  // same up to the fp32 accumulation order inside the matrix cores).
   const GemmPlan plan = plan_gemm(g, ws_bytes);
   const int shape = plan.shape;
   const bool pair_ok = pipe_ok && g.K % kQBK == 0;
-  if (pipe_ok && shape == 1)
-    launch_pipe<OutTag, 256, 128, 4, 3>(g, stream);
-  else if (pair_ok && shape == 0)
-    launch_pair<OutTag, 256, 256, 8>(g, stream);
-  else if (pair_ok && shape == 3 && one_round(g, 224, 256))
-    launch_pair<OutTag, 224, 256, 8, 3>(g, stream);
-  else if (pair_ok && shape == 3)
-    launch_pair<OutTag, 224, 256, 8>(g, stream);
-  else if (pipe_ok && shape == 0)
-    launch_pipe<OutTag, 256, 256, 8, 4>(g, stream);
-  else if (pipe_ok && shape == 3)
-    launch_pipe<OutTag, 224, 256, 8, 4>(g, stream);
-  else if (pipe_ok && shape == 4)
-    launch_pipe<OutTag, 224, 128, 4, 3>(g, stream);
-  else if (pair_ok && shape == 5)
+  if (pair_ok && shape == 5)
     launch_small<OutTag, 128, 128, 4, 4>(g, stream, plan.splits);
   else if (pair_ok && shape == 6)
     launch_small<OutTag, 64, 64, 4, 4>(g, stream, plan.splits);
-  else if (pair_ok && shape == 7)
-    launch_small<OutTag, 128, 256, 8, 3>(g, stream);
   else if (pair_ok && shape == 8)
     launch_small<OutTag, 64, 128, 4, 4>(g, stream);
-  else if (pair_ok && shape == 9)
-    launch_small<OutTag, 128, 192, 4, 3>(g, stream);
   else if (pair_ok && shape == 10)
     launch_small<OutTag, 128, 96, 4, 4, 4>(g, stream);
   else if (pair_ok && shape == 11)
     launch_small<OutTag, 64, 96, 2, 4, 2>(g, stream);
+  else if (pair_ok && shape >= kPair)
+    launch_pair_rows<OutTag>(g, stream, shape - kPair);
+  else if (pipe_ok && (shape >= kPair || launch_knob(JO_KNOB_GEMM_SHAPE) < 0) && pick_tile_rows(g.M, g.N) == 256)
+    launch_pipe<OutTag, 256, 256, 8, 4>(g, stream);
+  else if (pipe_ok && (shape >= kPair || launch_knob(JO_KNOB_GEMM_SHAPE) < 0))
+    launch_pipe<OutTag, 224, 256, 8, 4>(g, stream);
   else
     hipLaunchKernelGGL((fp8_gemm_kernel<OutTag>), grid, dim3(kBlock), 0, stream, g);
   return launch_status("fp8_scaled_mm");
