@@ -69,8 +69,9 @@ int jo_abi_version(void);
  *                       3 = 224x256, 4 = 160x256, 7 = 128x256 or 9 = 112x256;
  *                       5 = 128x128, 6 = 64x64, 8 = 64x128 and 10 = 128x96
  *                       (four waves), 11 = 64x96 (two waves); 2 = the
- *                       register-staged kernel, which also runs where 5-11
- *                       are forced and K % 128 != 0 (env JO_GEMM_SHAPE)
+ *                       register-staged kernel, which also runs for K == 0,
+ *                       scales_b not 16-byte or bias not 8-byte aligned, and
+ *                       256 operand rows of 4 GiB and more (env JO_GEMM_SHAPE)
  *   JO_KNOB_GEMM_SPLIT  FP8 GEMM K split: 1 (none), 2, 4 or 8 workgroups per
  *                       tile, taken by the 128x128 and 64x64 tiles when
  *                       jo_fp8_scaled_mm_ws has the workspace for it and

@@ -177,25 +177,6 @@ __global__ __launch_bounds__(kBlock, 1) void fp8_gemm_kernel(const GemmArgs g) {
   }
 }
 
-// ---------------------------------------------------------------------------
-// Pipelined kernel (K % 64 == 0): NW waves on a BM x BN tile (BM 256 or 224),
-// in a 2 x NW/2 grid of wave tiles 128 (or 96, the second row of a 224-row
-// tile) x 2*BN/NW (NW = 8: two waves per SIMD, so one wave's barrier and LDS
-// waits overlap the other's MFMAs). K advances in 64-byte stages through a
-// ring of NST LDS stages of (BM + BN) x 64 bytes filled by direct
-// global->LDS loads issued NST stages ahead, and each wave holds the
-// next stage's fragments in a second register set while the current stage's
-// MFMAs run. LDS rows are 64 bytes; chunk c of row r sits at chunk position
-// c ^ ((r >> 2) & 3). gfx950's LDS serves a ds_read_b128 sixteen lanes per
-// cycle from 64 four-byte banks: the sixteen consecutive rows a 16-lane group
-// reads then fall in sixteen distinct 16-byte bank groups (rocprofv3
-// SQ_LDS_BANK_CONFLICT reads 0 for this layout, 2.0e7 for an XOR with
-// ((r >> 1) ^ (r >> 3)) & 3, 6.1e7 unswizzled, on the 3120x16384x4096 GEMM).
-// ---------------------------------------------------------------------------
-constexpr int kPBK = 64;  // bytes of K per stage
-
-__device__ __forceinline__ int pswz(int r) { return (r >> 2) & 3; }
-
 // s_waitcnt limiting only the vector-memory counter to n (n < 64); s_waitcnt
 // limiting only the LDS counter to 0.
 #define JO_WAIT_VM(n) __builtin_amdgcn_s_waitcnt(0x0F70 | ((n) & 15) | (((n) >> 4) << 14))
@@ -213,314 +194,8 @@ __device__ __forceinline__ void wait_loads(int later) {
     JO_WAIT_VM(0);
 }
 
-// Direct loads of one stage: BM rows of A then BN rows of B^T, 64 bytes each,
-// written by (BM + BN) / 16 wave instructions of 1 KB (16 rows, four lanes per
-// row); slot L fills stage bytes L * 1024 .. +1024 and belongs to wave L % NW.
-template <int BM, int BN, int NW>
-struct PipeLoads {
-  static constexpr int kSlots = (BM + BN) / 16;
-  static constexpr int kPerWave = (kSlots + NW - 1) / NW;
-  static constexpr bool kEven = kSlots % NW == 0;
-  const uint8_t* base[kPerWave];  // wave-uniform: the tile's first row of A or B^T
-  uint32_t off[kPerWave];         // this lane's 16-byte chunk of each slot at K offset 0
-  bool last;                      // the wave owns a slot kPerWave - 1 (always when kEven)
-};
-
-// Epilogue of a wave's K loop, shared by the pipelined kernels. The LDS of
-// the K loop's ring (at least 128 padded output rows) is free once every wave
-// has passed the first barrier below.
-template <class OutTag, int BM, int BN, int NW, int MI>
-__device__ __forceinline__ void store_tile(const GemmArgs& g, uint8_t* smem,
-                                           const f32x16 (&acc)[MI][BN / (NW / 2) / 32], int wm,
-                                           int wn, int m0, int n0) {
-  constexpr int WCOLS = BN / (NW / 2);
-  constexpr int J = WCOLS / 32;
-  const int tid = threadIdx.x;
-  const int lane = tid % kWave;
-  const int fr = lane & 31, fh = lane >> 5;
-  // Subtile (i, j) element e of a lane is row
-  // m = m0 + wm*128 + i*32 + lane%32, column n = n0 + wn*WCOLS + j*32 +
-  // (e/4)*8 + (lane/32)*4 + e%4. The finished values go through LDS (free
-  // after the K loop) one 128-row half at a time, so that every row leaves
-  // as whole lines of 16-byte lane stores: stored straight from the MFMA
-  // layout (8 bytes per lane, 32 rows per wave store) the lines were written
-  // back part-filled, measured 2.4-4.5x the output bytes in WRITE_SIZE.
-  constexpr int kRowBytes = BN * 2 + 16;  // padded LDS row: 8-byte writes of 32 rows spread over the banks
-  float sam[MI];
-#pragma unroll
-  for (int i = 0; i < MI; ++i) sam[i] = g.sa[min(m0 + wm * 128 + i * 32 + fr, g.M - 1)];
-  float sbq[J][4][4], bq[J][4][4];
-#pragma unroll
-  for (int j = 0; j < J; ++j)
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int n = min(n0 + wn * WCOLS + j * 32 + q * 8 + fh * 4, g.N - 4);  // N % 8 == 0
-      const u32x4 sbv = ld16(g.sb + n);
-      u32x4 b4{0u, 0u, 0u, 0u};
-      if (g.bias) {
-        const u32x2 braw = *reinterpret_cast<const u32x2*>(static_cast<const uint16_t*>(g.bias) + n);
-        b4 = u32x4{braw.x, braw.y, 0u, 0u};
-      }
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        sbq[j][q][t] = elem<F32>(sbv, t);
-        bq[j][q][t] = g.bias ? elem<OutTag>(b4, t) : 0.f;
-      }
-    }
-  constexpr int kT = NW * 64;
-  constexpr int kChunksPerRow = BN * 2 / 16;
-#pragma unroll
-  for (int half = 0; half < 2; ++half) {
-    __syncthreads();  // the ring (or the previous half) is no longer read
-    if (wm == half) {
-#pragma unroll
-      for (int i = 0; i < MI; ++i)
-#pragma unroll
-        for (int j = 0; j < J; ++j)
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            float o[8];
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-              o[t] = __builtin_fmaf(sam[i], acc[i][j][q * 4 + t] * sbq[j][q][t], bq[j][q][t]);
-              o[t + 4] = 0.f;
-            }
-            const u32x4 pk = pack<OutTag>(o);
-            const int rl = i * 32 + fr, cl = wn * WCOLS + j * 32 + q * 8 + fh * 4;
-            *reinterpret_cast<u32x2*>(smem + rl * kRowBytes + cl * 2) = u32x2{pk.x, pk.y};
-          }
-    }
-    __syncthreads();
-    const int rows = half == 0 ? 128 : BM - 128;
-    for (int c = tid; c < rows * kChunksPerRow; c += kT) {
-      const int rl = c / kChunksPerRow, ch = c % kChunksPerRow;
-      const int m = m0 + half * 128 + rl, n = n0 + ch * 8;
-      if (m < g.M && n < g.N)
-        st16_nt(static_cast<uint16_t*>(g.out) + static_cast<int64_t>(m) * g.ldo + n,
-                *reinterpret_cast<const u32x4*>(smem + rl * kRowBytes + ch * 16));
-    }
-  }
-}
-
-// One output tile's K loop and epilogue for a wave holding MI row blocks of 32
-// (rows wm*128 .. wm*128 + 32*MI - 1 of the tile) and WCOLS columns.
-template <class OutTag, int BM, int BN, int NW, int NST, int MI>
-__device__ __forceinline__ void fp8_gemm_pipe_tile(const GemmArgs& g, uint8_t* smem,
-                                                   const PipeLoads<BM, BN, NW>& ld, int wave,
-                                                   int wm, int wn, int m0, int n0) {
-  using Loads = PipeLoads<BM, BN, NW>;
-  constexpr int WCOLS = BN / (NW / 2);  // wave tile columns
-  constexpr int J = WCOLS / 32;         // n-subtiles of 32 per wave
-  constexpr int kStage = (BM + BN) * kPBK;
-  static_assert(J >= 1 && MI >= 2 && MI <= 4, "tile shape");
-  const int tid = threadIdx.x;
-  const int lane = tid % kWave;
-  const int stages = g.K / kPBK;
-  auto issue = [&](int s) {
-    uint8_t* base = smem + (s % NST) * kStage;
-    const int kb = s * kPBK;
-#pragma unroll
-    for (int i = 0; i < Loads::kPerWave; ++i)
-      if (Loads::kEven || i + 1 < Loads::kPerWave || ld.last)
-        __builtin_amdgcn_global_load_lds(ld.base[i] + (ld.off[i] + kb), (__attribute__((address_space(3))) void*)(base + (wave + i * NW) * 1024), 16, 0, 0);
-  };
-
-  f32x16 acc[MI][J];
-#pragma unroll
-  for (int i = 0; i < MI; ++i)
-#pragma unroll
-    for (int j = 0; j < J; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
-
-  const int fr = lane & 31, fh = lane >> 5;
-  // LDS byte offsets of this lane's fragment chunks (same in every stage).
-  int offa[MI][2], offb[J][2];
-#pragma unroll
-  for (int i = 0; i < MI; ++i) {
-    const int r = wm * 128 + i * 32 + fr;
-#pragma unroll
-    for (int h = 0; h < 2; ++h) offa[i][h] = r * kPBK + (((fh * 2 + h) ^ pswz(r)) << 4);
-  }
-#pragma unroll
-  for (int j = 0; j < J; ++j) {
-    const int r = wn * WCOLS + j * 32 + fr;
-#pragma unroll
-    for (int h = 0; h < 2; ++h) offb[j][h] = BM * kPBK + r * kPBK + (((fh * 2 + h) ^ pswz(r)) << 4);
-  }
-
-  auto read_frags = [&](int s, i32x8 (&af)[MI], i32x8 (&bf)[J]) {
-    const uint8_t* st = smem + (s % NST) * kStage;
-#pragma unroll
-    for (int j = 0; j < J; ++j) {
-      const u32x4 lo = *reinterpret_cast<const u32x4*>(st + offb[j][0]);
-      const u32x4 hi = *reinterpret_cast<const u32x4*>(st + offb[j][1]);
-      bf[j] = i32x8{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
-    }
-#pragma unroll
-    for (int i = 0; i < MI; ++i) {
-      const u32x4 lo = *reinterpret_cast<const u32x4*>(st + offa[i][0]);
-      const u32x4 hi = *reinterpret_cast<const u32x4*>(st + offa[i][1]);
-      af[i] = i32x8{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
-    }
-  };
-  // Wait for this wave's loads of the stage being synced (with `later`
-  // younger stages still allowed in flight) and its LDS reads, then meet the
-  // other waves: that stage is complete in LDS, and every wave has finished
-  // reading the stage before it. A bare s_barrier: a fenced barrier would
-  // also wait for the loads of the later stages.
-  auto sync_stage = [&](int later) {
-    // On its own, outside the branch below: the compiler then knows that no
-    // LDS read is pending after it and lets the MFMAs of the current
-    // fragments run while the next stage's reads are in flight.
-    __builtin_amdgcn_sched_barrier(0);  // the waits stay after the previous stage's MFMAs
-    JO_WAIT_LDS0();
-    if (Loads::kEven || ld.last)
-      wait_loads<Loads::kPerWave>(later);
-    else
-      wait_loads<Loads::kPerWave - 1>(later);
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-  };
-
-  // Software pipeline: at the start of stage s the wave waits for its LDS
-  // reads (stage s's fragments) and for its own loads of stage s+1, then meets
-  // the other waves: stage s+1 is complete in LDS, and every wave holds its
-  // stage-s fragments, so the ring slot of stage s is free. It refills that
-  // slot with stage s+NST, starts reading stage s+1's fragments into the
-  // other register set and runs all of stage s's MFMAs while they arrive.
-  for (int s = 0; s < NST && s < stages; ++s) issue(s);
-  sync_stage(min(stages - 1, NST - 1));
-  i32x8 af0[MI], bf0[J], af1[MI], bf1[J];
-  read_frags(0, af0, bf0);
-  // B first: the accumulator is the transposed tile, so a lane holds one
-  // output row (m = lane % 32 of the subtile) and, per group of four
-  // registers, four consecutive columns — stored as one 8-byte chunk.
-  auto mfmas = [&](i32x8 (&af)[MI], i32x8 (&bf)[J]) {
-#pragma unroll
-    for (int i = 0; i < MI; ++i)
-#pragma unroll
-      for (int j = 0; j < J; ++j) acc[i][j] = mfma32(bf[j], af[i], acc[i][j]);
-  };
-  // While stage s+NST exists, NST-2 younger stages stay in flight at the
-  // sync: a constant wait.
-  auto steady = [&](int s, i32x8 (&af)[MI], i32x8 (&bf)[J], i32x8 (&an)[MI], i32x8 (&bn)[J]) {
-    // With 256-row tiles the first KB MFMAs of the stage go out before the
-    // barrier (their fragments are this wave's own), so the matrix cores are
-    // busy while the waves meet (4096^3: 67.4 -> 65.5 us on MI355X; with
-    // 224-row tiles it measured 1-2% slower and is not done).
-    constexpr int KB = BM == 256 ? 2 : 0;
-    if constexpr (KB > 0) {
-      __builtin_amdgcn_sched_barrier(0);
-      JO_WAIT_LDS0();
-      if (Loads::kEven || ld.last)
-        wait_loads<Loads::kPerWave>(NST - 2);
-      else
-        wait_loads<Loads::kPerWave - 1>(NST - 2);
-#pragma unroll
-      for (int q = 0; q < KB; ++q) acc[q / J][q % J] = mfma32(bf[q % J], af[q / J], acc[q / J][q % J]);
-      __builtin_amdgcn_sched_barrier(0);
-      asm volatile("" ::: "memory");
-      __builtin_amdgcn_s_barrier();
-      asm volatile("" ::: "memory");
-    } else {
-      sync_stage(NST - 2);
-    }
-    issue(s + NST);
-    read_frags(s + 1, an, bn);
-#pragma unroll
-    for (int q = KB; q < MI * J; ++q) acc[q / J][q % J] = mfma32(bf[q % J], af[q / J], acc[q / J][q % J]);
-    // Interleave: one MFMA, then two of the next stage's LDS reads (issuing
-    // every read first measured 5-10% slower than this order).
-#pragma unroll
-    for (int q = KB; q < MI * J; ++q) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
-      __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);  // DS read
-    }
-  };
-  auto drain = [&](int s, i32x8 (&af)[MI], i32x8 (&bf)[J], i32x8 (&an)[MI], i32x8 (&bn)[J]) {
-    if (s + 1 < stages) {
-      sync_stage(min(stages - 2 - s, NST - 2));
-      if (s + NST < stages) issue(s + NST);
-      read_frags(s + 1, an, bn);
-    }
-    mfmas(af, bf);
-  };
-  int s = 0;
-  for (; s + 1 + NST < stages; s += 2) {
-    steady(s, af0, bf0, af1, bf1);
-    steady(s + 1, af1, bf1, af0, bf0);
-  }
-  for (; s < stages; s += 2) {
-    drain(s, af0, bf0, af1, bf1);
-    if (s + 1 < stages) drain(s + 1, af1, bf1, af0, bf0);
-  }
-
-  static_assert(128 * (BN * 2 + 16) <= NST * kStage, "epilogue staging fits the ring");
-  store_tile<OutTag, BM, BN, NW, MI>(g, smem, acc, wm, wn, m0, n0);
-}
-
-template <class OutTag, int BM, int BN, int NW, int NST>
-__device__ __forceinline__ void fp8_gemm_pipe_body(const GemmArgs& g) {
-  using Loads = PipeLoads<BM, BN, NW>;
-  static_assert(BM == 256 || BM == 224, "tile rows");
-  __shared__ __attribute__((aligned(1024))) uint8_t smem[NST * (BM + BN) * kPBK];
-  const int tid = threadIdx.x;
-  const int lane = tid % kWave;
-  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
-  // BM = 256: a 2 x NW/2 grid of 128 x WCOLS wave tiles (even waves rows
-  // 0-127, odd waves rows 128-255). BM = 224: waves 0 .. NW/2-1 take rows
-  // 0-127 (four row blocks), the others rows 128-223 (three): a workgroup's
-  // waves are spread round-robin over the CU's four SIMDs, so with NW = 8
-  // each SIMD runs one wave of each kind, 7 row blocks where a 256-row tile
-  // gives it 8.
-  const int wm = BM == 256 ? (wave & 1) : wave / (NW / 2);
-  const int wn = BM == 256 ? (wave >> 1) : wave % (NW / 2);
-  const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
-
-  // Lane p of a slot fills row +p/4, chunk position p%4 with the global chunk
-  // that belongs there. Rows beyond M (N) read row M-1 (N-1); they are never
-  // stored. Addresses are a wave-uniform 64-bit tile base plus a 32-bit lane
-  // offset (the host keeps 256 rows of A and B^T under 4 GB), which saves the
-  // VGPRs of 64-bit per-lane pointers.
-  Loads ld;
-#pragma unroll
-  for (int i = 0; i < Loads::kPerWave; ++i) {
-    const int slot = wave + i * NW;
-    const bool is_a = slot < BM / 16;
-    const int r = (is_a ? slot : slot - BM / 16) * 16 + lane / 4;
-    const int row = is_a ? min(m0 + r, g.M - 1) - m0 : min(n0 + r, g.N - 1) - n0;
-    ld.base[i] = is_a ? g.a + static_cast<int64_t>(m0) * g.lda : g.b + static_cast<int64_t>(n0) * g.ldb;
-    ld.off[i] = static_cast<uint32_t>(row) * static_cast<uint32_t>(is_a ? g.lda : g.ldb) +
-                (((lane & 3) ^ pswz(r)) * 16);
-  }
-  ld.last = Loads::kEven || wave + (Loads::kPerWave - 1) * NW < Loads::kSlots;
-  if constexpr (BM == 256) {
-    fp8_gemm_pipe_tile<OutTag, BM, BN, NW, NST, 4>(g, smem, ld, wave, wm, wn, m0, n0);
-  } else {
-    if (wm == 0)
-      fp8_gemm_pipe_tile<OutTag, BM, BN, NW, NST, 4>(g, smem, ld, wave, wm, wn, m0, n0);
-    else
-      fp8_gemm_pipe_tile<OutTag, BM, BN, NW, NST, 3>(g, smem, ld, wave, wm, wn, m0, n0);
-  }
-}
-
-// The body lives in a device function: with the lambdas above directly in a
-// kernel template over NW, the host compiler emits no launch stub for it.
-template <class OutTag, int BM, int BN, int NW, int NST>
-__global__ __launch_bounds__(NW * 64, 8 / NW) void fp8_gemm_pipe_kernel(const GemmArgs g) {
-  fp8_gemm_pipe_body<OutTag, BM, BN, NW, NST>(g);
-}
-
-template <class OutTag, int BM, int BN, int NW, int NST>
-void launch_pipe(const GemmArgs& g, hipStream_t stream) {
-  hipLaunchKernelGGL((fp8_gemm_pipe_kernel<OutTag, BM, BN, NW, NST>),
-                     dim3((g.N + BN - 1) / BN, (g.M + BM - 1) / BM), dim3(NW * 64), 0, stream, g);
-}
-
 // ---------------------------------------------------------------------------
-// Pair kernel (K % 128 == 0), the default for many rows: eight waves on a
+// Pair kernel, the default for many rows: eight waves on a
 // BM x 256 tile (BM a multiple of 16 from 96 to 256), two per SIMD, in a 2 x 4
 // grid of wave tiles of 64 columns whose first row takes (BM / 16 + 1) / 2 of
 // the 16-row blocks. K advances in 128-byte stages, one
@@ -564,6 +239,28 @@ __device__ __forceinline__ void static_for(Fn&& fn) {
   }
 }
 
+// A K that is not a multiple of 128 (it is one of 16): the part of a stage that
+// is left over at its end is taken first, so that the loops know nothing of
+// it. Chunks past K read that stage's first chunk of their row instead (always
+// inside the row), and A's are then zeroed in LDS by the lanes that loaded
+// them: what B holds there is multiplied by zero (it is a value of the same
+// row of B, so a NaN among them was in the sum already). The lane's chunk
+// position is the same in every load slot of a wave: slots are NW apart (even)
+// and A has an even number of them.
+struct KTail {
+  bool part;       // K is not whole stages
+  int back;        // bytes from this lane's chunk back to the row's first, if its chunk is past K
+  uint32_t first;  // K offset of stage 0's loads, from operand bases moved back by shift()
+  __device__ __forceinline__ KTail(int K, int lane, int wave) {
+    const int bytes = (K - 1) % kQBK + 1, pos = ((lane & 7) ^ qswz((wave & 1) * 8 + lane / 8)) * 16;
+    part = bytes != kQBK;
+    back = pos >= bytes ? pos : 0;
+    first = part ? static_cast<uint32_t>((K + kQBK - 1) / kQBK * kQBK - back) : 0u;
+  }
+  // Stage t >= 1 then reads from t * 128 on: whole stage t - 1 if stage 0 is the part.
+  __device__ __forceinline__ int shift() const { return part ? kQBK : 0; }
+};
+
 // Direct loads of one stage: BM rows of A then BN rows of B^T, 128 bytes
 // each, written by (BM + BN) / 8 wave instructions of 1 KB (8 rows, eight
 // lanes per row); slot L fills stage bytes L * 1024 .. +1024 and belongs to
@@ -593,7 +290,7 @@ constexpr int pair_ring_bytes() {
 // two, so B loads run NBS - 1 stages ahead and A loads one.
 template <class OutTag, int BM, int BN, int NW, int MI, int NBS>
 __device__ __forceinline__ void fp8_gemm_pair_tile(const GemmArgs& g, uint8_t* smem,
-                                                   const PairLoads<BM, BN, NW>& ld, int wave,
+                                                   const PairLoads<BM, BN, NW>& ld, const KTail& kt, int wave,
                                                    int row0, int wn, int m0, int n0) {
   using Loads = PairLoads<BM, BN, NW>;
   constexpr int WCOLS = BN / (NW / 2);  // wave tile columns
@@ -610,7 +307,7 @@ __device__ __forceinline__ void fp8_gemm_pair_tile(const GemmArgs& g, uint8_t* s
   constexpr int kScaleOff = pair_ring_bytes<BM, BN, NW, NBS>();
   static_assert((NBS == 2 || NBS == 3) && (BN / 8) % NW == 0, "B ring");
   const int lane = threadIdx.x % kWave;
-  const int stages = g.K / kQBK;
+  const int stages = (g.K + kQBK - 1) / kQBK;
   // Load i of this wave is A (slot index below BM / 8; a wave's A loads come
   // first in its slot order) or B: known at compile time but for the one index
   // that the last A slots share with the first B slots.
@@ -620,22 +317,22 @@ __device__ __forceinline__ void fp8_gemm_pair_tile(const GemmArgs& g, uint8_t* s
     if constexpr (i * NW >= BM / 8) return false;
     return wave + i * NW < BM / 8;
   };
-  // Load i of stage t, A to slot t % 2 and B to ring slot bslot.
-  auto issue_one = [&](int t, int bslot, auto ic) {
+  // Load i of stage t at K offset koff, A to slot t % 2 and B to ring slot bslot.
+  auto issue_one = [&](int t, int bslot, uint32_t koff, auto ic) {
     constexpr int i = decltype(ic)::value;
     if (Loads::kEven || i + 1 < PER || ld.last) {
       uint8_t* dst = is_a(ic) || NBS == 2 ? smem + (t & 1) * kASlot + (wave + i * NW) * 1024
                                           : smem + kBBase + bslot * kBSlot + (wave + i * NW - BM / 8) * 1024;
-      __builtin_amdgcn_global_load_lds(ld.base[i] + (ld.off[i] + t * kQBK), (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
+      __builtin_amdgcn_global_load_lds(ld.base[i] + (ld.off[i] + koff), (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
     }
   };
   // The loads issued in stage s's second half: A of stage s + 2 and B of
   // stage s + NBS, the latter into the slot of stage s's B (bcur).
   auto issue_batch_one = [&](int s, int bcur, auto ic) {
     if (NBS == 2 || is_a(ic))
-      issue_one(s + 2, 0, ic);
+      issue_one(s + 2, 0, (s + 2) * kQBK, ic);
     else if (s + NBS < stages)
-      issue_one(s + NBS, bcur, ic);
+      issue_one(s + NBS, bcur, (s + NBS) * kQBK, ic);
   };
 
   f32x4 acc[MI][J];
@@ -747,10 +444,12 @@ __device__ __forceinline__ void fp8_gemm_pair_tile(const GemmArgs& g, uint8_t* s
   // within a stage); stage 0 starts once its own loads are in.
   auto issue_part = [&](int t, bool a) {
     static_for<PER>([&](auto ic) {
-      if (is_a(ic) == a) issue_one(t, t, ic);
+      if (is_a(ic) == a) issue_one(t, t, t == 0 ? kt.first : t * kQBK, ic);
     });
   };
-  auto issue = [&](int t) { static_for<PER>([&](auto ic) { issue_one(t, t, ic); }); };
+  auto issue = [&](int t) {
+    static_for<PER>([&](auto ic) { issue_one(t, t, t == 0 ? kt.first : t * kQBK, ic); });
+  };
   // The tile's scales and bias go to LDS first (4 bytes a lane, 64 lanes a
   // load), the oldest loads of all, so that the epilogue does not start with
   // a wait for memory.
@@ -802,6 +501,14 @@ __device__ __forceinline__ void fp8_gemm_pair_tile(const GemmArgs& g, uint8_t* s
       JO_WAIT_LDS0();
       JO_WAIT_VM(0);
     }
+  }
+  if (kt.part) {  // this wave's loads of stage 0 are in
+    asm volatile("" ::: "memory");
+    if (kt.back)
+      static_for<PER>([&](auto ic) {
+        if (is_a(ic)) *reinterpret_cast<u32x4*>(smem + (wave + decltype(ic)::value * NW) * 1024 + lane * 16) = u32x4{0u, 0u, 0u, 0u};
+      });
+    JO_WAIT_LDS0();
   }
   bare_barrier();
 #pragma unroll
@@ -926,25 +633,26 @@ __device__ __forceinline__ void fp8_gemm_pair_body(const GemmArgs& g) {
   // stored. Wave-uniform 64-bit tile bases plus 32-bit lane offsets (the host
   // keeps 256 rows of A and B^T under 4 GB).
   Loads ld;
+  const KTail kt(g.K, lane, wave);
 #pragma unroll
   for (int i = 0; i < Loads::kPerWave; ++i) {
     const int slot = wave + i * NW;
     const bool is_a = slot < BM / 8;
     const int r = (is_a ? slot : slot - BM / 8) * 8 + lane / 8;
     const int row = is_a ? min(m0 + r, g.M - 1) - m0 : min(n0 + r, g.N - 1) - n0;
-    ld.base[i] = is_a ? g.a + static_cast<int64_t>(m0) * g.lda : g.b + static_cast<int64_t>(n0) * g.ldb;
+    ld.base[i] = (is_a ? g.a + static_cast<int64_t>(m0) * g.lda : g.b + static_cast<int64_t>(n0) * g.ldb) - kt.shift();
     ld.off[i] = static_cast<uint32_t>(row) * static_cast<uint32_t>(is_a ? g.lda : g.ldb) +
                 (((lane & 7) ^ qswz(r)) * 16);
   }
   ld.last = Loads::kEven || wave + (Loads::kPerWave - 1) * NW < Loads::kSlots;
   constexpr int kUp = (RB + 1) / 2, kLow = RB / 2;
   if constexpr (kUp == kLow) {
-    fp8_gemm_pair_tile<OutTag, BM, BN, NW, kUp, NBS>(g, smem, ld, wave, wm * kUp * 16, wn, m0, n0);
+    fp8_gemm_pair_tile<OutTag, BM, BN, NW, kUp, NBS>(g, smem, ld, kt, wave, wm * kUp * 16, wn, m0, n0);
   } else {
     if (wm == 0)
-      fp8_gemm_pair_tile<OutTag, BM, BN, NW, kUp, NBS>(g, smem, ld, wave, 0, wn, m0, n0);
+      fp8_gemm_pair_tile<OutTag, BM, BN, NW, kUp, NBS>(g, smem, ld, kt, wave, 0, wn, m0, n0);
     else
-      fp8_gemm_pair_tile<OutTag, BM, BN, NW, kLow, NBS>(g, smem, ld, wave, kUp * 16, wn, m0, n0);
+      fp8_gemm_pair_tile<OutTag, BM, BN, NW, kLow, NBS>(g, smem, ld, kt, wave, kUp * 16, wn, m0, n0);
   }
 }
 
@@ -1034,25 +742,26 @@ __device__ __forceinline__ void fp8_gemm_small_body(const GemmArgs& g) {
   // rows), chunk position p%8, with the global chunk that belongs there; rows
   // beyond M (N) read row M-1 (N-1) and are never stored.
   Loads ld;
+  const KTail kt(g.K, lane, wave);
 #pragma unroll
   for (int i = 0; i < PER; ++i) {
     const int slot = wave + i * NW;
     const bool is_a = slot < BM / 8;
     const int r = (is_a ? slot : slot - BM / 8) * 8 + lane / 8;
     const int row = is_a ? min(m0 + r, g.M - 1) - m0 : min(n0 + r, g.N - 1) - n0;
-    ld.base[i] = is_a ? g.a + static_cast<int64_t>(m0) * g.lda : g.b + static_cast<int64_t>(n0) * g.ldb;
+    ld.base[i] = (is_a ? g.a + static_cast<int64_t>(m0) * g.lda : g.b + static_cast<int64_t>(n0) * g.ldb) - kt.shift();
     ld.off[i] = static_cast<uint32_t>(row) * static_cast<uint32_t>(is_a ? g.lda : g.ldb) +
                 (((lane & 7) ^ qswz(r)) * 16);
   }
   // SPLIT: workgroup z of the grid's gridDim.z takes the z-th equal share of
   // the K stages and writes its partial product for the reduction kernel.
-  const int stages = SPLIT ? g.K / kQBK / static_cast<int>(gridDim.z) : g.K / kQBK;
+  const int stages = SPLIT ? g.K / kQBK / static_cast<int>(gridDim.z) : (g.K + kQBK - 1) / kQBK;
   const int s0 = SPLIT ? static_cast<int>(blockIdx.z) * stages : 0;
   auto issue = [&](int s) {
     uint8_t* dst = smem + (s % NST) * kStage;
 #pragma unroll
     for (int i = 0; i < PER; ++i)
-      __builtin_amdgcn_global_load_lds(ld.base[i] + (ld.off[i] + (s0 + s) * kQBK),
+      __builtin_amdgcn_global_load_lds(ld.base[i] + (ld.off[i] + (!SPLIT && s == 0 ? kt.first : static_cast<uint32_t>((s0 + s) * kQBK))),
                                        (__attribute__((address_space(3))) void*)(dst + (wave + i * NW) * 1024),
                                        16, 0, 0);
   };
@@ -1111,6 +820,13 @@ __device__ __forceinline__ void fp8_gemm_small_body(const GemmArgs& g) {
     JO_WAIT_LDS0();
     wait_loads<PER>(min(stages - 1 - s, NST - 2));
     asm volatile("" ::: "memory");
+    if (!SPLIT && s == 0 && kt.part) {  // a split K is whole stages
+      if (kt.back)
+#pragma unroll
+        for (int i = 0; i < PER; ++i)
+          if (wave + i * NW < BM / 8) *reinterpret_cast<u32x4*>(smem + (wave + i * NW) * 1024 + lane * 16) = u32x4{0u, 0u, 0u, 0u};
+      JO_WAIT_LDS0();
+    }
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     if (s + NST - 1 < stages) issue(s + NST - 1);
@@ -1330,13 +1046,6 @@ int auto_shape(int cus, int M, int N) {
   return shape;
 }
 
-// Pair tile rows where K is not whole 128-byte stages (the 64-byte-stage kernel).
-int pick_tile_rows(int M, int N) {
-  const int64_t cus = cu_count(), cols = (N + 255) / 256;
-  auto cost = [&](int64_t bm) { return ((M + bm - 1) / bm * cols + cus - 1) / cus * (bm / 32); };
-  return cost(224) < cost(256) ? 224 : 256;
-}
-
 // Split K, for few tiles and a long K (the text stream's MLP down: [256,
 // 16384] x [16384, 4096] is 64 tiles of 128x128): S workgroups share each
 // tile's K stages and write fp32 partials that a second kernel adds up in a
@@ -1419,31 +1128,26 @@ int launch_gemm(const GemmArgs& g, hipStream_t stream, int64_t ws_bytes) {
   const dim3 grid((g.N + kBN - 1) / kBN, (g.M + kBM - 1) / kBM);
   // K == 0 takes the register-staged kernel, which loads no operand bytes
   // when K is 0 and stores the epilogue of a zero accumulator (the bias).
-  const bool pipe_ok = g.K > 0 && g.K % kPBK == 0 && aligned(g.sb, 16) && (g.bias == nullptr || aligned(g.bias, 8)) &&
-                       256 * (g.lda > g.ldb ? g.lda : g.ldb) + g.K <= int64_t{UINT32_MAX};
+  const bool direct_ok = g.K > 0 && aligned(g.sb, 16) && (g.bias == nullptr || aligned(g.bias, 8)) &&
+                         256 * (g.lda > g.ldb ? g.lda : g.ldb) + g.K <= int64_t{UINT32_MAX};
   // The JO_KNOB_GEMM_SHAPE override forces a shape (knob_shape; results are the
   // same up to the fp32 accumulation order inside the matrix cores).
   const GemmPlan plan = plan_gemm(g, ws_bytes);
   const int shape = plan.shape;
-  const bool pair_ok = pipe_ok && g.K % kQBK == 0;
-  if (pair_ok && shape == 5)
-    launch_small<OutTag, 128, 128, 4, 4>(g, stream, plan.splits);
-  else if (pair_ok && shape == 6)
-    launch_small<OutTag, 64, 64, 4, 4>(g, stream, plan.splits);
-  else if (pair_ok && shape == 8)
-    launch_small<OutTag, 64, 128, 4, 4>(g, stream);
-  else if (pair_ok && shape == 10)
-    launch_small<OutTag, 128, 96, 4, 4, 4>(g, stream);
-  else if (pair_ok && shape == 11)
-    launch_small<OutTag, 64, 96, 2, 4, 2>(g, stream);
-  else if (pair_ok && shape >= kPair)
-    launch_pair_rows<OutTag>(g, stream, shape - kPair);
-  else if (pipe_ok && (shape >= kPair || launch_knob(JO_KNOB_GEMM_SHAPE) < 0) && pick_tile_rows(g.M, g.N) == 256)
-    launch_pipe<OutTag, 256, 256, 8, 4>(g, stream);
-  else if (pipe_ok && (shape >= kPair || launch_knob(JO_KNOB_GEMM_SHAPE) < 0))
-    launch_pipe<OutTag, 224, 256, 8, 4>(g, stream);
-  else
+  if (!direct_ok || shape == 2)
     hipLaunchKernelGGL((fp8_gemm_kernel<OutTag>), grid, dim3(kBlock), 0, stream, g);
+  else if (shape == 5)
+    launch_small<OutTag, 128, 128, 4, 4>(g, stream, plan.splits);
+  else if (shape == 6)
+    launch_small<OutTag, 64, 64, 4, 4>(g, stream, plan.splits);
+  else if (shape == 8)
+    launch_small<OutTag, 64, 128, 4, 4>(g, stream);
+  else if (shape == 10)
+    launch_small<OutTag, 128, 96, 4, 4, 4>(g, stream);
+  else if (shape == 11)
+    launch_small<OutTag, 64, 96, 2, 4, 2>(g, stream);
+  else
+    launch_pair_rows<OutTag>(g, stream, shape - kPair);
   return launch_status("fp8_scaled_mm");
 }
 
