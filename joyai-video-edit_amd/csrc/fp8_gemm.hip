@@ -972,6 +972,193 @@ void launch_small(const GemmArgs& args, hipStream_t stream, int splits = 1) {
                      dim3(kBlock), 0, stream, g, splits);
 }
 
+// ---------------------------------------------------------------------------
+// Streaming kernel, for up to 80 rows: the weight is read once and that is
+// what the time should go to. A workgroup of eight waves takes BM = 16 MB rows
+// (all of them) x BN = 16 NB columns, so one wave's fragments are used by no
+// other; its waves split K instead, wave w taking the 128-byte steps w, w + 8,
+// ... of every row. Each brings its steps through an LDS region of its own
+// (direct loads of whole lines, the pair kernel's row layout) and waits for
+// nothing but its own loads: there is no barrier in the loop, and the other
+// waves' loads are in flight meanwhile. The partial tiles meet in LDS at the
+// end and are added in wave order (the same bits on every run).
+// Measured against the small-tile kernel, us, weights from HBM / cached:
+// 16x4096x4096 11.7 -> 6.8 (HBM), 40x4096x4096 12.2 -> 8.3, 77x4096x4096 12.1
+// -> 10.2 / 10.4 -> 8.3, 77x12288x4096 17.4 -> 16.9 / 15.8 -> 12.3,
+// 77x16384x4096 19.2 -> 20.3 / 15.5 -> 14.9 (left to it), 1x12288x4096 13.3 -> 11.7 /
+// 10.3 -> 9.9, 24x3072x3072 9.9 -> 5.6 / 8.3 -> 3.9. About 4 us of it are the launch, the first loads' latency and the
+// last exchange; at 77 rows every workgroup also reads 320 KB of A from its L2.
+// Fragments loaded straight into registers in MFMA layout (64 bytes a row and
+// load instead of whole lines) measured 20.4 / 17.8 at 77x12288x4096;
+// nontemporal loads of B 14.9 / 14.3 (77x16384x4096 18.2 / 17.7): nothing of the
+// weight is then found in the Infinity Cache on a repeat.
+// ---------------------------------------------------------------------------
+constexpr int kStreamLds = 152 * 1024;
+
+constexpr int kStreamWaves = 8;
+constexpr int kStreamRows = 80;
+
+template <int MB, int NB>
+struct StreamShape {
+  static constexpr int NW = kStreamWaves;
+  static constexpr int kPitch = NB * 16 + 4;                 // floats of a staged row
+  static constexpr int kBlock = NW * 16 * kPitch * 4;        // bytes of a staged row block
+  static constexpr int kPass = kStreamLds / kBlock < MB ? kStreamLds / kBlock : MB;
+  static constexpr int kStep = (MB + NB) * 2048;             // bytes of a wave's step
+  static constexpr int kMain = NW * kStep > kPass * kBlock ? NW * kStep : kPass * kBlock;
+  static constexpr int kScales = MB * 16 * 4 + NB * 16 * 4 + NB * 16 * 2;
+  static_assert(NW * kStep <= kStreamLds && kMain + 1024 + kScales <= 160 * 1024, "LDS");
+};
+
+template <int MB, int NB>
+__device__ __forceinline__ void fp8_gemm_stream_body(const GemmArgs& g, int out_bf16) {
+  using Sh = StreamShape<MB, NB>;
+  constexpr int NW = kStreamWaves;
+  constexpr int BN = NB * 16;
+  __shared__ __attribute__((aligned(1024))) uint8_t smem[Sh::kMain + Sh::kScales];
+  const int tid = threadIdx.x;
+  const int lane = tid % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int fr = lane & 15, fh = lane >> 4;
+  const int n0 = blockIdx.x * BN;
+  const int steps = g.K / kQBK, left = g.K % kQBK;  // whole steps, bytes of a last, partial one
+
+  // Lane p of load slot L fills row 8 L + p / 8 of the step (A rows, then B^T
+  // rows), chunk position p % 8, with the global chunk that belongs there.
+  // Rows past M (N) read row M - 1 (N - 1) and are never stored.
+  uint8_t* mine = smem + wave * Sh::kStep;
+  uint32_t off[(MB + NB) * 2];
+#pragma unroll
+  for (int i = 0; i < (MB + NB) * 2; ++i) {
+    const int r = (i < MB * 2 ? i : i - MB * 2) * 8 + lane / 8;
+    const int row = i < MB * 2 ? min(r, g.M - 1) : min(n0 + r, g.N - 1) - n0;
+    off[i] = static_cast<uint32_t>(row) * static_cast<uint32_t>(i < MB * 2 ? g.lda : g.ldb) +
+             (((lane & 7) ^ qswz(r)) * 16);
+  }
+  const uint8_t* pb = g.b + static_cast<int64_t>(n0) * g.ldb;
+  auto issue = [&](int s) {
+#pragma unroll
+    for (int i = 0; i < (MB + NB) * 2; ++i) {
+      // A chunk past K reads the row's first chunk of the step.
+      const int c = ((lane & 7) ^ qswz((i & 1) * 8 + lane / 8)) * 16;
+      const uint32_t k = s * kQBK - (s == steps && c >= left ? c : 0);
+      __attribute__((address_space(3))) void* dst = (__attribute__((address_space(3))) void*)(mine + i * 1024);
+      __builtin_amdgcn_global_load_lds((i < MB * 2 ? g.a : pb) + (off[i] + k), dst, 16, 0, 0);
+    }
+  };
+  // Scales and bias, the oldest loads of the last wave.
+  uint8_t* scales = smem + Sh::kMain;
+  if (wave == NW - 1) {
+    auto load4 = [&](const void* src, int at) {
+      __builtin_amdgcn_global_load_lds(static_cast<const uint8_t*>(src), (__attribute__((address_space(3))) void*)(scales + at), 4, 0, 0);
+    };
+#pragma unroll
+    for (int r = 0; r < MB * 16; r += kWave)
+      if (r + lane < MB * 16) load4(g.sa + min(r + lane, g.M - 1), r * 4);
+    if (lane < BN) load4(g.sb + min(n0 + lane, g.N - 1), MB * 64);
+    if (g.bias && lane < BN / 2) load4(static_cast<const uint16_t*>(g.bias) + min(n0 + lane * 2, g.N - 2), MB * 64 + BN * 4);
+  }
+
+  f32x4 acc[MB][NB];
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  int at[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) at[h] = fr * kQBK + (((fh * 2 + h) ^ qswz(fr)) << 4);
+  const int all = steps + (left != 0 ? 1 : 0);
+  if (wave < all) issue(wave);
+  for (int s = wave; s < all; s += NW) {
+    JO_WAIT_VM(0);
+    asm volatile("" ::: "memory");
+    i32x8 af[MB], bf[NB];
+    auto frag = [&](int block) {
+      const u32x4 lo = *reinterpret_cast<const u32x4*>(mine + block * 2048 + at[0]);
+      const u32x4 hi = *reinterpret_cast<const u32x4*>(mine + block * 2048 + at[1]);
+      return i32x8{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
+    };
+#pragma unroll
+    for (int j = 0; j < NB; ++j) bf[j] = frag(MB + j);
+#pragma unroll
+    for (int i = 0; i < MB; ++i) af[i] = frag(i);
+    if (s == steps) {  // A past K: zero
+#pragma unroll
+      for (int i = 0; i < MB; ++i)
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          if ((fh * 2 + e / 4) * 16 >= left) af[i][e] = 0;
+    }
+    // The fragments are held before the region is filled again.
+    JO_WAIT_LDS0();
+    asm volatile("" ::: "memory");
+    if (s + NW < all) issue(s + NW);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+      for (int j = 0; j < NB; ++j) acc[i][j] = mfma16(bf[j], af[i], acc[i][j]);
+  }
+  JO_WAIT_VM(0);  // a wave without steps may have loaded scales
+
+  // Lane: row i*16 + lane%16 of the tile, columns j*16 + (lane/16)*4 .. +3.
+  constexpr int kQuads = BN / 4;
+  constexpr int kPlane = Sh::kPass * 16 * Sh::kPitch;
+  float* part = reinterpret_cast<float*>(smem);
+#pragma unroll
+  for (int i0 = 0; i0 < MB; i0 += Sh::kPass) {
+    __syncthreads();  // every wave is done with its region, or the previous pass
+#pragma unroll
+    for (int i = i0; i < i0 + Sh::kPass && i < MB; ++i)
+#pragma unroll
+      for (int j = 0; j < NB; ++j)
+        *reinterpret_cast<f32x4*>(part + wave * kPlane + ((i - i0) * 16 + fr) * Sh::kPitch + j * 16 + fh * 4) = acc[i][j];
+    __syncthreads();
+    const int rows = (MB - i0 < Sh::kPass ? MB - i0 : Sh::kPass) * 16;
+    for (int c = tid; c < rows * kQuads; c += NW * kWave) {
+      const int r = c / kQuads, col = c % kQuads * 4, n = n0 + col, m = i0 * 16 + r;
+      if (m >= g.M || n >= g.N) continue;
+      const float* p = part + r * Sh::kPitch + col;
+      f32x4 v = *reinterpret_cast<const f32x4*>(p);
+#pragma unroll
+      for (int w = 1; w < NW; ++w) v += *reinterpret_cast<const f32x4*>(p + w * kPlane);
+      {
+        const float sa = *reinterpret_cast<const float*>(scales + (i0 * 16 + r) * 4);
+        const u32x4 sbv = *reinterpret_cast<const u32x4*>(scales + MB * 64 + col * 4);
+        const u32x2 braw = *reinterpret_cast<const u32x2*>(scales + MB * 64 + BN * 4 + col * 2);
+        const u32x4 b4{braw.x, braw.y, 0u, 0u};
+        float o[8];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          const float bias = !g.bias ? 0.f : out_bf16 ? elem<BF16>(b4, t) : elem<F16>(b4, t);
+          o[t] = __builtin_fmaf(sa, v[t] * elem<F32>(sbv, t), bias);
+          o[t + 4] = 0.f;
+        }
+        const u32x4 pk = out_bf16 ? pack<BF16>(o) : pack<F16>(o);
+        *reinterpret_cast<u32x2*>(static_cast<uint16_t*>(g.out) + static_cast<int64_t>(m) * g.ldo + n) = u32x2{pk.x, pk.y};
+      }
+    }
+  }
+}
+
+template <int MB, int NB>
+__global__ __launch_bounds__(kStreamWaves * 64, 1) void fp8_gemm_stream_kernel(const GemmArgs g, int out_bf16) {
+  fp8_gemm_stream_body<MB, NB>(g, out_bf16);
+}
+
+// The kernel of mb x nb row and column blocks.
+template <int MB = kStreamRows / 16, int NB = 4>
+void launch_stream(const GemmArgs& g, int mb, int nb, int bf16, hipStream_t stream) {
+  if constexpr (MB > 1) {
+    if (mb < MB) return launch_stream<MB - 1, NB>(g, mb, nb, bf16, stream);
+  }
+  if constexpr (NB > 1) {
+    if (nb < NB) return launch_stream<MB, NB - 1>(g, mb, nb, bf16, stream);
+  }
+  hipLaunchKernelGGL((fp8_gemm_stream_kernel<MB, NB>), dim3((g.N + NB * 16 - 1) / (NB * 16)),
+                     dim3(kStreamWaves * 64), 0, stream, g, bf16);
+}
+
 // CUs of the current device (queried once per device; 256, MI355X's count,
 // if the query fails).
 int cu_count() {
@@ -989,7 +1176,9 @@ int cu_count() {
 // Launch shapes. kPair + rows: the eight-wave pair kernel with tiles of that
 // many rows x 256 columns (a multiple of 16 from 96 to 256); 2: the
 // register-staged kernel; 5, 6, 8, 10, 11: the small-tile kernel.
+// kStream + 16 NB: the streaming kernel with NB column blocks.
 constexpr int kPair = 1000;
+constexpr int kStream = 2000;
 
 // Cost of a pair-kernel launch and of a small-tile one in the same unit, a
 // small-tile kernel's operand bytes per K byte on the busiest CU (those run at
@@ -1060,6 +1249,18 @@ int auto_shape(int cus, int M, int N) {
 // unsplit (16.5 us; split in two, 20.6).
 constexpr int64_t kSplitCap = int64_t{1} << 30;  // largest partial buffer a split uses
 
+// Estimated time of the streaming kernel, ns: the launch, first loads and last
+// exchange; every row of A once a workgroup out of L2 (109 KB/us a CU); and B
+// at what HBM gives all CUs (5.0 TB/s) or a CU can draw (33 KB/us). Fitted to
+// M = 1, 16, 40 and 77 at N = 4096 to 16384, mostly within 15% of what was
+// measured.
+int64_t stream_ns(int cus, int M, int N, int K, int nb) {
+  const int64_t tiles = (N + nb * 16 - 1) / (nb * 16), rounds = (tiles + cus - 1) / cus;
+  const int64_t a = rounds * ((M + 15) / 16 * 16) * K / 109;
+  const int64_t b = static_cast<int64_t>(N) * K / 5000, b_cu = rounds * nb * 16 * K / 33;
+  return 3000 + a + (b > b_cu ? b : b_cu);
+}
+
 struct GemmPlan {
   int shape;
   int splits;
@@ -1120,7 +1321,31 @@ GemmPlan plan_gemm(const GemmArgs& g, int64_t ws_bytes) {
           split = GemmPlan{c[0], sp};
         }
       }
-  return (best >= 0 && best * 20 < unsplit * 17) ? split : p;
+  const bool splits = best >= 0 && best * 20 < unsplit * 17;
+  if (splits) p = split;
+  // Few rows: the streaming kernel where it is estimated faster than the
+  // choice so far, which takes 3 us and its operand bytes at 49 KB/us a CU; with
+  // a split, 4 us more for the second launch, and 75 KB/us where workgroups
+  // share a CU.
+  if (g.M <= kStreamRows) {
+    int64_t other = 3000 + unsplit / 49;
+    if (splits) {
+      const int64_t t = split.shape == 5 ? 128 : 64;
+      const int64_t wgs = (g.M + t - 1) / t * ((g.N + t - 1) / t) * split.splits, per = (wgs + cus - 1) / cus;
+      other = 7000 + per * 2 * t * (g.K / split.splits) / (per > 1 ? 75 : 49);
+    }
+    for (int nb = 1; nb <= 4; ++nb) {
+      const int64_t ns = stream_ns(cus, g.M, g.N, g.K, nb);
+      // On a tie up to 32 rows take the wider tile (fewer workgroups' fixed
+      // cost: 1x12288x4096 12.1 / 10.3 us with three column blocks, 11.7 / 9.9
+      // with four), above the narrower one (at 77 rows 16.9 / 12.5 and 17.8 / 12.6).
+      if (ns < other || (ns == other && p.shape >= kStream && g.M <= 32)) {
+        other = ns;
+        p = GemmPlan{kStream + nb * 16, 1};
+      }
+    }
+  }
+  return p;
 }
 
 template <class OutTag>
@@ -1146,8 +1371,10 @@ int launch_gemm(const GemmArgs& g, hipStream_t stream, int64_t ws_bytes) {
     launch_small<OutTag, 128, 96, 4, 4, 4>(g, stream);
   else if (shape == 11)
     launch_small<OutTag, 64, 96, 2, 4, 2>(g, stream);
-  else
+  else if (shape < kStream)
     launch_pair_rows<OutTag>(g, stream, shape - kPair);
+  else
+    launch_stream(g, (g.M + 15) / 16, (shape - kStream) / 16, std::is_same<OutTag, BF16>::value, stream);
   return launch_status("fp8_scaled_mm");
 }
 
