@@ -858,6 +858,154 @@ torch::Tensor fp8_scaled_mm(const torch::Tensor& mat_a, const torch::Tensor& mat
   return out;
 }
 
+// ---------------------------------------------------------------------------
+// The DiT's calls (joyomni_ops/dit_ops.py) as one dispatch each: the reshapes,
+// output allocations and launches that the Python shims made one by one (at a
+// few rows a call's time was that host work: an Fp8Linear 16 us, of which the
+// two kernels take 7).
+// ---------------------------------------------------------------------------
+namespace {
+// Whether x [..., H, D] has a contiguous last dim and leading dims that
+// collapse to one token stride (what rmsnorm_heads reads without a copy).
+bool heads_view(const torch::Tensor& x) {
+  if (x.dim() < 2 || (x.stride(-1) != 1 && x.size(-1) > 1)) return false;
+  int64_t next = -1;
+  for (int64_t d = x.dim() - 3; d >= 0; --d) {
+    if (x.size(d) == 1) continue;
+    if (next >= 0 && x.stride(d) != next) return false;
+    next = x.stride(d) * x.size(d);
+  }
+  return true;
+}
+
+// A modulation vector as the fused norm ops take it, without copies: [B, D] or
+// [B, 1, D] -> [B, D] ([D] when B == 1), [B, L, D] -> [B * L, D].
+torch::Tensor mod_per_sample(const torch::Tensor& t, int64_t B, int64_t L, int64_t D) {
+  if (t.numel() == B * D) return B == 1 ? t.reshape({D}) : t.reshape({B, D});
+  return t.reshape({B * L, D});
+}
+
+std::tuple<torch::Tensor, torch::Tensor> fp8_outputs(const torch::Tensor& x, int64_t M, int64_t K) {
+  return {torch::empty({M, K}, x.options().dtype(at::kFloat8_e4m3fn)),
+          torch::empty({M, 1}, x.options().dtype(torch::kFloat32))};
+}
+
+// q or k [B, L, H, D] as the tables op reads it where it is: contiguous heads,
+// whole 16-byte rows of tokens that do not overlap.
+bool token_rows(const torch::Tensor& x) {
+  if (x.dim() != 4 || !x.is_cuda() || x.scalar_type() != torch::kBFloat16 || x.numel() == 0) return false;
+  const int64_t D = x.size(3), row = x.size(2) * D;
+  return (D == 64 || D == 128 || D == 256) && x.stride(3) == 1 && x.stride(2) == D &&
+         x.stride(1) >= row && x.stride(1) % 8 == 0 &&
+         (x.size(0) == 1 || (x.stride(0) >= 0 && x.stride(0) % 8 == 0)) &&
+         reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0;
+}
+
+// A table [1, L, D], [1, L, D/2] or without the leading 1, as the tables op
+// reads it; undefined if it is anything else.
+torch::Tensor table32(const torch::Tensor& t, const torch::Tensor& q) {
+  if (t.scalar_type() != torch::kFloat32 || t.device() != q.device()) return {};
+  const torch::Tensor v = t.dim() == 3 && t.size(0) == 1 ? t.select(0, 0) : t;
+  const int64_t L = q.size(1), D = q.size(3);
+  if (v.dim() != 2 || v.size(0) != L || (v.size(1) != D && v.size(1) != D / 2) || v.stride(1) != 1 ||
+      v.stride(0) % 4 != 0 || v.stride(0) < v.size(1) ||
+      reinterpret_cast<uintptr_t>(v.data_ptr()) % 16 != 0)
+    return {};
+  return v;
+}
+
+bool direct_tables(const torch::Tensor& q, const torch::Tensor& k, torch::Tensor& cos,
+                   torch::Tensor& sin) {
+  if (!token_rows(q) || !token_rows(k) || q.sizes() != k.sizes()) return false;
+  cos = table32(cos, q);
+  sin = table32(sin, q);
+  return cos.defined() && sin.defined() && cos.sizes() == sin.sizes() && cos.strides() == sin.strides();
+}
+}  // namespace
+
+std::tuple<torch::Tensor, torch::Tensor> quantize_activation(const torch::Tensor& x) {
+  const torch::Tensor x2 = x.reshape({-1, x.size(-1)}).contiguous();
+  auto [q, s] = fp8_outputs(x2, x2.size(0), x2.size(1));
+  sgl_per_token_quant_fp8(x2, q, s);
+  return {q, s};
+}
+
+std::tuple<torch::Tensor, torch::Tensor> gelu_quantize_activation(const torch::Tensor& h) {
+  torch::Tensor h2 = h.reshape({-1, h.size(-1)});
+  if (h2.stride(-1) != 1) h2 = h2.contiguous();
+  auto [q, s] = fp8_outputs(h2, h2.size(0), h2.size(1));
+  gelu_tanh_quant_fp8(h2, q, s, c10::nullopt);
+  return {q, s};
+}
+
+torch::Tensor fp8_linear(const torch::Tensor& x, const torch::Tensor& weight,
+                         const torch::Tensor& weight_scale, const c10::optional<torch::Tensor>& bias,
+                         at::ScalarType out_dtype) {
+  auto [q, s] = quantize_activation(x);
+  const torch::Tensor y = fp8_scaled_mm(q, weight, s, weight_scale, out_dtype, bias);
+  std::vector<int64_t> shape(x.sizes().begin(), x.sizes().end());
+  shape.back() = weight.size(1);
+  return y.reshape(shape);
+}
+
+torch::Tensor layernorm_modulate(const torch::Tensor& x, const c10::optional<torch::Tensor>& gamma,
+                                 const c10::optional<torch::Tensor>& beta, const torch::Tensor& scale,
+                                 const torch::Tensor& shift, double eps) {
+  TORCH_CHECK(x.dim() == 3, "x must be [B, L, D]");
+  const int64_t B = x.size(0), L = x.size(1), D = x.size(2);
+  return fused_norm_scale_shift_per_sample(x.reshape({-1, D}), gamma, beta,
+                                           mod_per_sample(scale, B, L, D),
+                                           mod_per_sample(shift, B, L, D), 0, eps)
+      .reshape({B, L, D});
+}
+
+std::tuple<torch::Tensor, torch::Tensor> add_gate_layernorm_modulate_fp8(
+    const torch::Tensor& x, const c10::optional<torch::Tensor>& residual,
+    const c10::optional<torch::Tensor>& gate, const c10::optional<torch::Tensor>& gamma,
+    const c10::optional<torch::Tensor>& beta, const torch::Tensor& scale, const torch::Tensor& shift,
+    double eps) {
+  TORCH_CHECK(x.dim() == 3, "x must be [B, L, D]");
+  const int64_t B = x.size(0), L = x.size(1), D = x.size(2);
+  auto [q, s] = fp8_outputs(x, B * L, D);
+  c10::optional<torch::Tensor> res, g;
+  if (residual.has_value()) res = residual->view({B * L, D});
+  if (gate.has_value()) g = mod_per_sample(*gate, B, L, D);
+  norm_scale_shift_quant_fp8(x.reshape({B * L, D}), res, g, gamma, beta,
+                             mod_per_sample(scale, B, L, D), mod_per_sample(shift, B, L, D), 0, eps,
+                             q, s);
+  return {q, s};
+}
+
+// RMSNorm over the last dim: heads in place where the view allows it, else a
+// contiguous copy (round_first as rmsnorm_heads).
+torch::Tensor rmsnorm_last(const torch::Tensor& x, const torch::Tensor& weight, double eps,
+                           int64_t round_first) {
+  if (heads_view(x)) return rmsnorm_heads(x, weight, eps, round_first);
+  const int64_t D = x.size(-1);
+  if (round_first) return rmsnorm_heads(x.reshape({-1, 1, D}).contiguous(), weight, eps, 1).reshape(x.sizes());
+  return rmsnorm(x.reshape({-1, D}).contiguous(), weight, eps).reshape(x.sizes());
+}
+
+// (q, k) from the tables op where it takes these forms of q, k and the tables
+// and neither q nor k is contiguous (those are rotated in place), else nothing.
+std::vector<torch::Tensor> qk_norm_rope_direct(const torch::Tensor& q, const torch::Tensor& k, double eps,
+                                               const torch::Tensor& q_weight,
+                                               const torch::Tensor& k_weight, torch::Tensor cos,
+                                               torch::Tensor sin) {
+  if (q.is_contiguous() || k.is_contiguous() || !direct_tables(q, k, cos, sin)) return {};
+  auto out = fused_qk_norm_rope_3d_tables(q, k, q.size(1), q.size(2), eps, q_weight, k_weight, cos, sin);
+  return {std::get<0>(out), std::get<1>(out)};
+}
+
+bool qk_norm_rope_kstage_direct(torch::Tensor& q, torch::Tensor& k, torch::Tensor& k_stage, double eps,
+                                const torch::Tensor& q_weight, const torch::Tensor& k_weight,
+                                torch::Tensor cos, torch::Tensor sin) {
+  if (!direct_tables(q, k, cos, sin)) return false;
+  fused_qk_norm_rope_3d_tables_kstage(q, k, k_stage, q.size(1), q.size(2), eps, q_weight, k_weight, cos,
+                                      sin);
+  return true;
+}
+
 }  // namespace joyomni_ops
 
 TORCH_LIBRARY(joyomni_ops, m) {
@@ -916,6 +1064,24 @@ TORCH_LIBRARY(joyomni_ops, m) {
   m.def(
       "fused_norm_scale_shift_per_sample(Tensor x, Tensor? gamma_opt, Tensor? beta_opt, "
       "Tensor scale, Tensor shift, int norm_type, float eps) -> Tensor");
+  m.def("quantize_activation(Tensor x) -> (Tensor, Tensor)");
+  m.def("gelu_quantize_activation(Tensor h) -> (Tensor, Tensor)");
+  m.def(
+      "fp8_linear(Tensor x, Tensor weight, Tensor weight_scale, Tensor? bias, ScalarType out_dtype) "
+      "-> Tensor");
+  m.def(
+      "layernorm_modulate(Tensor x, Tensor? gamma, Tensor? beta, Tensor scale, Tensor shift, "
+      "float eps) -> Tensor");
+  m.def(
+      "add_gate_layernorm_modulate_fp8(Tensor x, Tensor(a!)? residual, Tensor? gate, Tensor? gamma, "
+      "Tensor? beta, Tensor scale, Tensor shift, float eps) -> (Tensor, Tensor)");
+  m.def("rmsnorm_last(Tensor x, Tensor weight, float eps, int round_first) -> Tensor");
+  m.def(
+      "qk_norm_rope_direct(Tensor q, Tensor k, float eps, Tensor q_weight, Tensor k_weight, "
+      "Tensor cos, Tensor sin) -> Tensor[]");
+  m.def(
+      "qk_norm_rope_kstage_direct(Tensor(a!) q, Tensor(b!) k, Tensor(c!) k_stage, float eps, "
+      "Tensor q_weight, Tensor k_weight, Tensor cos, Tensor sin) -> bool");
 }
 
 TORCH_LIBRARY_IMPL(joyomni_ops, CUDA, m) {
@@ -939,4 +1105,12 @@ TORCH_LIBRARY_IMPL(joyomni_ops, CUDA, m) {
   m.impl("apply_rotary_emb", &joyomni_ops::apply_rotary_emb);
   m.impl("rmsnorm_heads", &joyomni_ops::rmsnorm_heads);
   m.impl("fused_norm_scale_shift_per_sample", &joyomni_ops::fused_norm_scale_shift_per_sample);
+  m.impl("quantize_activation", &joyomni_ops::quantize_activation);
+  m.impl("gelu_quantize_activation", &joyomni_ops::gelu_quantize_activation);
+  m.impl("fp8_linear", &joyomni_ops::fp8_linear);
+  m.impl("layernorm_modulate", &joyomni_ops::layernorm_modulate);
+  m.impl("add_gate_layernorm_modulate_fp8", &joyomni_ops::add_gate_layernorm_modulate_fp8);
+  m.impl("rmsnorm_last", &joyomni_ops::rmsnorm_last);
+  m.impl("qk_norm_rope_direct", &joyomni_ops::qk_norm_rope_direct);
+  m.impl("qk_norm_rope_kstage_direct", &joyomni_ops::qk_norm_rope_kstage_direct);
 }

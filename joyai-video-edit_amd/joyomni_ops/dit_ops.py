@@ -49,12 +49,22 @@ from typing import Optional, Sequence, Tuple
 
 import torch
 
-from . import (fp8_scaled_mm, fused_add_layernorm_scale_shift, fused_norm_scale_shift,
-               fused_norm_scale_shift_per_sample, fused_qk_norm_rope_3d_grid, fused_qk_norm_rope_3d_grid_kstage, gelu_tanh_quant_fp8,
-               fused_qk_norm_rope_3d_paired, fused_qk_norm_rope_3d_paired_kstage,
-               fused_qk_norm_rope_3d_tables, fused_qk_norm_rope_3d_tables_kstage,
-               kv_commit_rope, norm_scale_shift_quant_fp8, rmsnorm, rmsnorm_heads,
-               rope_freqs, sgl_per_token_quant_fp8)
+from . import (fp8_scaled_mm, fused_add_layernorm_scale_shift, fused_qk_norm_rope_3d_grid,
+               fused_qk_norm_rope_3d_paired, fused_qk_norm_rope_3d_paired_kstage, kv_commit_rope,
+               rope_freqs)
+
+# One dispatch per call: the reshapes, output allocations and launches of these
+# calls are made inside the op (at a few rows they are what a call costs: an
+# Fp8Linear of 12 rows 16 us from Python, its two kernels 6).
+_ops = torch.ops.joyomni_ops
+_quantize_activation = _ops.quantize_activation.default
+_gelu_quantize_activation = _ops.gelu_quantize_activation.default
+_fp8_linear = _ops.fp8_linear.default
+_layernorm_modulate = _ops.layernorm_modulate.default
+_add_gate_layernorm_modulate_fp8 = _ops.add_gate_layernorm_modulate_fp8.default
+_rmsnorm_last = _ops.rmsnorm_last.default
+_qk_norm_rope_direct = _ops.qk_norm_rope_direct.default
+_qk_norm_rope_kstage_direct = _ops.qk_norm_rope_kstage_direct.default
 
 
 def available() -> bool:
@@ -77,11 +87,7 @@ def fused_layernorm_modulate(
     Per-sample vectors are read in place, one row per sample of L tokens
     (fused_norm_scale_shift_per_sample), for any B: no [B*L, D] expanded
     copies; per-token modulation is read a row each."""
-    B, L, D = x.shape
-    out = fused_norm_scale_shift_per_sample(x.reshape(-1, D), weight, bias,
-                                            _mod_per_sample(scale, B, L, D),
-                                            _mod_per_sample(shift, B, L, D), "layer", eps)
-    return out.reshape(B, L, D)
+    return _layernorm_modulate(x, weight, bias, scale, shift, eps)
 
 
 def fused_qk_norm_rope_3d(
@@ -102,14 +108,14 @@ def fused_qk_norm_rope_3d(
     if q.dtype != torch.bfloat16:
         raise RuntimeError(f"fused_qk_norm_rope_3d requires bf16 q/k, got {q.dtype}")
     B, L, H, D = q.shape
-    if not (q.is_contiguous() or k.is_contiguous()) and _token_rows(q) and _token_rows(k):
+    if not (torch.is_grad_enabled() and (q.requires_grad or k.requires_grad)):
         # Strided slices and fp32 tables: one pass from where they are
         # ([1, 3120, 32, 128] of a packed qkv: 50.4 -> 19.3 us on MI355X against
         # the copies of q and k, the four table kernels and the paired op).
-        tables = _fp32_tables(freqs_cis, L, D, q.device)
-        if tables is not None:
-            return fused_qk_norm_rope_3d_tables(q, k, L, H, eps, q_norm_weight.to(torch.bfloat16),
-                                                k_norm_weight.to(torch.bfloat16), *tables)
+        out = _qk_norm_rope_direct(q, k, eps, _bf16(q_norm_weight), _bf16(k_norm_weight),
+                                   freqs_cis[0], freqs_cis[1])
+        if out:
+            return out[0], out[1]
     q = q.contiguous()
     k = k.contiguous()
     q_r = q.view(B, L * H, D)
@@ -121,33 +127,8 @@ def fused_qk_norm_rope_3d(
     return q, k
 
 
-def _token_rows(x: torch.Tensor) -> bool:
-    """x [B, L, H, D] as the strided QK ops read it without a copy: contiguous
-    heads, whole 16-byte rows of tokens that do not overlap, nothing recorded by autograd."""
-    B, L, H, D = x.shape
-    sb, sl, sh, sd = x.stride()
-    return (x.dtype == torch.bfloat16 and x.is_cuda and D in (64, 128, 256) and sd == 1 and sh == D
-            and sl >= H * D and sl % 8 == 0 and (B == 1 or (sb >= 0 and sb % 8 == 0))
-            and x.numel() > 0 and x.data_ptr() % 16 == 0
-            and not (x.requires_grad and torch.is_grad_enabled()))
-
-
-def _fp32_tables(freqs_cis, L: int, D: int, device):
-    """(cos, sin) as [L, D] or [L, D/2] views for the ops that read fp32 tables in
-    place, or None if they are anything else (which _half_tables_bf16 converts)."""
-    cos, sin = freqs_cis
-    shape = cos.shape
-    if len(shape) == 3 and shape[0] == 1:
-        cos, shape = cos[0], shape[1:]
-    if sin.dim() == 3 and sin.shape[0] == 1:
-        sin = sin[0]
-    if (len(shape) != 2 or shape[0] != L or shape[1] not in (D, D // 2) or sin.shape != shape
-            or cos.dtype != torch.float32 or sin.dtype != torch.float32 or cos.device != device
-            or sin.device != device or cos.stride() != sin.stride() or cos.stride(1) != 1
-            or cos.stride(0) % 4 or cos.stride(0) < shape[1] or cos.data_ptr() % 16
-            or sin.data_ptr() % 16):
-        return None
-    return cos, sin
+def _bf16(w: torch.Tensor) -> torch.Tensor:
+    return w if w.dtype is torch.bfloat16 else w.to(torch.bfloat16)
 
 
 def _half_tables_bf16(freqs_cis, L: int, D: int, device):
@@ -195,34 +176,17 @@ def fused_qk_norm_rope_3d_kstage(
     B, L, H, D = q.shape
     if k_stage is None:
         k_stage = torch.empty((B, L, H, D), dtype=torch.bfloat16, device=q.device)
-    if _token_rows(q) and _token_rows(k):
-        tables = _fp32_tables(freqs_cis, L, D, q.device)
-        if tables is not None:  # the fp32 tables are read as they are
-            fused_qk_norm_rope_3d_tables_kstage(q, k, k_stage, L, H, eps,
-                                                q_norm_weight.to(torch.bfloat16).contiguous(),
-                                                k_norm_weight.to(torch.bfloat16).contiguous(),
-                                                *tables)
+    if not (torch.is_grad_enabled() and (q.requires_grad or k.requires_grad)):
+        # fp32 tables are read as they are
+        if _qk_norm_rope_kstage_direct(q, k, k_stage, eps, _bf16(q_norm_weight).contiguous(),
+                                       _bf16(k_norm_weight).contiguous(), freqs_cis[0],
+                                       freqs_cis[1]):
             return q, k, k_stage
     cos, sin = _half_tables_bf16(freqs_cis, L, D, q.device)
     fused_qk_norm_rope_3d_paired_kstage(q, k, k_stage, L, H, eps,
                                         q_norm_weight.to(torch.bfloat16).contiguous(),
                                         k_norm_weight.to(torch.bfloat16).contiguous(), cos, sin)
     return q, k, k_stage
-
-
-def _heads_view(x: torch.Tensor) -> bool:
-    """x [..., H, D] with a contiguous last dim whose leading dims collapse to
-    one token stride (what rmsnorm_heads reads without a copy)."""
-    if x.dim() < 2 or (x.stride(-1) != 1 and x.shape[-1] > 1):
-        return False
-    nxt = None
-    for d in range(x.dim() - 3, -1, -1):
-        if x.shape[d] == 1:
-            continue
-        if nxt is not None and x.stride(d) != nxt:
-            return False
-        nxt = x.stride(d) * x.shape[d]
-    return True
 
 
 def rmsnorm_qk_bf16(x: torch.Tensor, weight: torch.Tensor, eps: float = 1e-6) -> torch.Tensor:
@@ -233,13 +197,7 @@ def rmsnorm_qk_bf16(x: torch.Tensor, weight: torch.Tensor, eps: float = 1e-6) ->
     new contiguous tensor of x's shape, bit-identical to the rmsnorm op on the
     copy (same kernel, same summation order)."""
     assert x.dtype == torch.bfloat16, f"rmsnorm_qk_bf16 needs bf16, got {x.dtype}"
-    w = weight.to(dtype=torch.bfloat16)
-    if _heads_view(x):
-        return rmsnorm_heads(x, w, eps)
-    orig_shape = x.shape
-    D = orig_shape[-1]
-    out = rmsnorm(x.reshape(-1, D).contiguous(), w, eps)
-    return out.reshape(orig_shape)
+    return _rmsnorm_last(x, _bf16(weight), eps, 0)
 
 
 def rms_norm_module(x: torch.Tensor, weight: Optional[torch.Tensor] = None,
@@ -254,10 +212,7 @@ def rms_norm_module(x: torch.Tensor, weight: Optional[torch.Tensor] = None,
         weight = torch.ones(D, dtype=x.dtype, device=x.device)
     if weight.dtype != x.dtype:
         raise RuntimeError(f"rms_norm_module: weight dtype {weight.dtype} != x dtype {x.dtype}")
-    if _heads_view(x):
-        return rmsnorm_heads(x, weight, eps, round_first=True)
-    return rmsnorm_heads(x.reshape(-1, 1, D).contiguous(), weight, eps,
-                         round_first=True).reshape(x.shape)
+    return _rmsnorm_last(x, weight, eps, 1)
 
 
 def fused_add_gate(residual: torch.Tensor, x: torch.Tensor, gate: torch.Tensor) -> torch.Tensor:
@@ -331,12 +286,7 @@ def fused_qk_norm_rope_3d_grid_views(
 def quantize_activation_fp8(x: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
     """The activation side of Fp8Linear.forward (fp8_linear.py:140-144, 166):
     x [..., K] -> (x_q fp8 e4m3fn [M, K], x_scale fp32 [M, 1]) with M = numel / K."""
-    x_2d = x.reshape(-1, x.shape[-1]).contiguous()
-    M, K = x_2d.shape
-    x_q = torch.empty((M, K), device=x_2d.device, dtype=torch.float8_e4m3fn)
-    x_scale = torch.empty((M, 1), device=x_2d.device, dtype=torch.float32)
-    sgl_per_token_quant_fp8(x_2d, x_q, x_scale)
-    return x_q, x_scale
+    return _quantize_activation(x)
 
 
 def gelu_quantize_activation_fp8(h: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
@@ -345,13 +295,7 @@ def gelu_quantize_activation_fp8(h: torch.Tensor) -> Tuple[torch.Tensor, torch.T
     next Fp8Linear.forward, fp8_linear.py:140-166): h [..., K] bf16/fp16 ->
     (x_q fp8 e4m3fn [M, K], x_scale fp32 [M, 1]). The activation is evaluated
     in fp32 and rounded to h's dtype before it is quantized, as the two calls do."""
-    h_2d = h.reshape(-1, h.shape[-1])
-    if h_2d.stride(-1) != 1:
-        h_2d = h_2d.contiguous()
-    M, K = h_2d.shape
-    x_q, x_scale = _fp8_outputs(M, K, h_2d.device)
-    gelu_tanh_quant_fp8(h_2d, x_q, x_scale)
-    return x_q, x_scale
+    return _gelu_quantize_activation(h)
 
 
 def _mod_per_sample(t: torch.Tensor, B: int, L: int, D: int) -> torch.Tensor:
@@ -361,12 +305,6 @@ def _mod_per_sample(t: torch.Tensor, B: int, L: int, D: int) -> torch.Tensor:
     if t.numel() == B * D:
         return t.reshape(D) if B == 1 else t.reshape(B, D)
     return t.reshape(B * L, D)
-
-
-def _fp8_outputs(M: int, D: int, device) -> Tuple[torch.Tensor, torch.Tensor]:
-    """x_q fp8 e4m3fn [M, D] and x_scale fp32 [M, 1], as Fp8Linear.forward allocates them."""
-    return (torch.empty((M, D), device=device, dtype=torch.float8_e4m3fn),
-            torch.empty((M, 1), device=device, dtype=torch.float32))
 
 
 def layernorm_modulate_fp8(
@@ -381,12 +319,7 @@ def layernorm_modulate_fp8(
     """quantize_activation_fp8(fused_layernorm_modulate(x, shift, scale)) in one
     pass: x [B, L, D], shift/scale [B, D], [B, 1, D] or [B, L, D] ->
     (x_q [B*L, D], x_scale [B*L, 1]), byte-identical to the two calls."""
-    B, L, D = x.shape
-    x_q, x_scale = _fp8_outputs(B * L, D, x.device)
-    norm_scale_shift_quant_fp8(x.reshape(B * L, D), _mod_per_sample(scale, B, L, D),
-                               _mod_per_sample(shift, B, L, D), x_q, x_scale, gamma=weight,
-                               beta=bias, eps=eps)
-    return x_q, x_scale
+    return _add_gate_layernorm_modulate_fp8(x, None, None, weight, bias, scale, shift, eps)
 
 
 def fused_add_gate_layernorm_modulate_fp8(
@@ -403,15 +336,10 @@ def fused_add_gate_layernorm_modulate_fp8(
     """fused_add_gate_layernorm_modulate followed by quantize_activation_fp8 of
     its modulated output, in one pass: returns (residual', x_q [B*L, D],
     x_scale [B*L, 1]); residual [B, L, D] is updated in place."""
-    B, L, D = x.shape
     if not residual.is_contiguous():
         raise RuntimeError("residual must be contiguous (it is updated in place)")
-    x_q, x_scale = _fp8_outputs(B * L, D, x.device)
-    norm_scale_shift_quant_fp8(x.reshape(B * L, D), _mod_per_sample(scale, B, L, D),
-                               _mod_per_sample(shift, B, L, D), x_q, x_scale,
-                               residual=residual.view(B * L, D),
-                               gate=_mod_per_sample(gate, B, L, D), gamma=weight, beta=bias,
-                               eps=eps)
+    x_q, x_scale = _add_gate_layernorm_modulate_fp8(x, residual, gate, weight, bias, scale, shift,
+                                                    eps)
     return residual, x_q, x_scale
 
 
@@ -444,9 +372,7 @@ def fp8_linear(x: torch.Tensor, weight_fp8: torch.Tensor, weight_scale: torch.Te
                bias: Optional[torch.Tensor] = None, out_dtype=torch.bfloat16) -> torch.Tensor:
     """Fp8Linear.forward (fp8_linear.py:155-169): x [..., K] bf16 -> per-token
     fp8 + scales -> fp8_scaled_mm with the per-channel weight scales and bias."""
-    x_q, x_scale = quantize_activation_fp8(x)
-    y = fp8_scaled_mm(x_q, weight_fp8, x_scale, weight_scale, out_dtype, bias)
-    return y.reshape(*x.shape[:-1], weight_fp8.shape[1])
+    return _fp8_linear(x, weight_fp8, weight_scale, bias, out_dtype)
 
 
 def fp8_linear_quantized(x_q: torch.Tensor, x_scale: torch.Tensor, weight_fp8: torch.Tensor,
