@@ -328,6 +328,125 @@ __global__ __launch_bounds__(kBlock) void norm_mod_kernel(const NormArgs a) {
   }
 }
 
+// One row per workgroup in 8-byte chunks of four 16-bit elements, held in
+// registers: rows whose length (or stride) is a multiple of 4 but not of 8,
+// which the ops take and the 16-byte row kernel does not. CH chunks a thread,
+// N <= 1024 CH. Bound like the row kernel by the row's bytes, at half its width
+// a load; the element-wise kernel that took these rows reads them three times,
+// two bytes a lane: LayerNorm + AdaLN of [3120, 3076] 21.9 -> 11.0 us, [3120,
+// 8188] 70.5 -> 21.6 ([3120, 3072] through the row kernel: 8.9).
+template <class Tag, int NT, bool ADD, bool QNT, int CH>
+__global__ __launch_bounds__(kBlock) void norm_mod_quad_kernel(const NormArgs a) {
+  __shared__ float red[kBlock / kWave];
+  const int64_t row = blockIdx.x;
+  const int N = a.N, quads = N / 4;
+  const int64_t mrow = mod_row(a, row);
+  auto load4 = [](const void* p, int64_t i, float (&o)[4]) {
+    const u32x2 w = *reinterpret_cast<const u32x2*>(static_cast<const uint16_t*>(p) + i);
+    const u32x4 c{w.x, w.y, 0u, 0u};
+#pragma unroll
+    for (int t = 0; t < 4; ++t) o[t] = elem<Tag>(c, t);
+  };
+  auto store4 = [](void* p, int64_t i, const float (&v)[4]) {
+    const float w[8] = {v[0], v[1], v[2], v[3], 0.f, 0.f, 0.f, 0.f};
+    const u32x4 c = pack<Tag>(w);
+    *reinterpret_cast<u32x2*>(static_cast<uint16_t*>(p) + i) = u32x2{c.x, c.y};
+  };
+  // Chunks past the row read its first one and are left out of every sum, the
+  // maximum and the stores.
+  auto at = [&](int c, bool& ok) {
+    const int i = threadIdx.x + c * kBlock;
+    ok = i < quads;
+    return (ok ? i : 0) * 4;
+  };
+  float v[CH][4];
+  float sum = 0.f;
+#pragma unroll
+  for (int c = 0; c < CH; ++c) {
+    bool ok;
+    const int e = at(c, ok);
+    load4(a.x, row * a.xs + e, v[c]);
+    if constexpr (ADD) {
+      float res[4], gate[4] = {1.f, 1.f, 1.f, 1.f};
+      load4(a.res, row * a.rs + e, res);
+      if (a.gate) load4(a.gate, mrow * a.gs + e, gate);
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+        v[c][t] = round_to<Tag>(residual_update(res[t], v[c][t], gate[t], a.gate != nullptr));
+    }
+#pragma unroll
+    for (int t = 0; t < 4; ++t) sum += !ok ? 0.f : NT == kLayer ? v[c][t] : v[c][t] * v[c][t];
+  }
+  if constexpr (ADD) {
+    __syncthreads();  // threads past the row have read its first chunk
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+      bool ok;
+      const int e = at(c, ok);
+      if (ok) store4(a.res, row * a.rs + e, v[c]);
+    }
+  }
+  sum = block_reduce<OpSum>(sum, red);
+  float mean = 0.f, r;
+  if constexpr (NT == kLayer) {
+    mean = div_by_len(sum, N);
+    float ss = 0.f;
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+      bool ok;
+      at(c, ok);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const float d = v[c][t] - mean;
+        ss += ok ? d * d : 0.f;
+      }
+    }
+    ss = block_reduce<OpSum>(ss, red);
+    r = 1.0f / sqrtf(div_by_len(ss, N) + a.eps);
+  } else {
+    r = 1.0f / sqrtf(div_by_len(sum, N) + a.eps);
+  }
+  const bool affine = a.gamma != nullptr;
+  const bool has_beta = affine && a.beta != nullptr && NT == kLayer;
+  float amax = 0.f;
+#pragma unroll
+  for (int c = 0; c < CH; ++c) {
+    bool ok;
+    const int e = at(c, ok);
+    float sc[4], sh[4], ga[4] = {1.f, 1.f, 1.f, 1.f}, be[4] = {0.f, 0.f, 0.f, 0.f};
+    load4(a.scale, mrow * a.scs + e, sc);
+    load4(a.shift, mrow * a.shs + e, sh);
+    if (affine) load4(a.gamma, e, ga);
+    if (has_beta) load4(a.beta, e, be);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      float y = (NT == kLayer) ? (v[c][t] - mean) * r : v[c][t] * r;
+      if (affine) y = y * ga[t];
+      if (has_beta) y = y + be[t];
+      y = y * (1.f + sc[t]) + sh[t];
+      v[c][t] = QNT ? round_to<Tag>(y) : y;
+      if (QNT && ok) amax = fmaxf(amax, fabsf(v[c][t]));
+    }
+    if constexpr (!QNT)
+      if (ok) store4(a.y, row * a.ys + e, v[c]);
+  }
+  if constexpr (QNT) {
+    amax = block_reduce<OpAmax>(amax, red);
+    const float scale = amax / kFp8Max;
+    if (threadIdx.x == 0) a.s[row] = scale;
+    const float inv = (scale == 0.f) ? 0.f : 1.0f / scale;
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+      bool ok;
+      const int e = at(c, ok);
+      uint32_t w = 0;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) w |= static_cast<uint32_t>(fp8_byte(v[c][t] * inv)) << (8 * t);
+      if (ok) *reinterpret_cast<uint32_t*>(a.q + row * a.qs + e) = w;
+    }
+  }
+}
+
 // One row per workgroup with element-wise accesses (any N, any alignment).
 // With QNT, y is evaluated twice (for the row maximum, then to quantize):
 // both evaluations are the same operations on the same values.
@@ -437,6 +556,31 @@ int launch_norm_mod(const NormArgs& a, hipStream_t stream, const char* op) {
                            stream, a);
       }
     }, a.M);
+  }
+  if constexpr (Tag::kVec == 8) {
+    bool quad_ok = !launched && a.N % 4 == 0 && a.N <= 16 * 4 * kBlock && aligned(a.x, 8) &&
+                   a.xs % 4 == 0 && aligned(a.scale, 8) && a.scs % 4 == 0 && aligned(a.shift, 8) &&
+                   a.shs % 4 == 0 && aligned(a.gamma, 8) && aligned(a.beta, 8) &&
+                   (QNT ? aligned(a.q, 4) && a.qs % 4 == 0 : aligned(a.y, 8) && a.ys % 4 == 0);
+    if (ADD) quad_ok = quad_ok && aligned(a.res, 8) && a.rs % 4 == 0 && aligned(a.gate, 8) && a.gs % 4 == 0;
+    if (quad_ok) {
+      auto go = [&](auto ch) {
+        hipLaunchKernelGGL((norm_mod_quad_kernel<Tag, NT, ADD, QNT, decltype(ch)::value>), dim3(a.M),
+                           dim3(kBlock), 0, stream, a);
+      };
+      const int64_t ch = (a.N / 4 + kBlock - 1) / kBlock;
+      if (ch <= 1)
+        go(std::integral_constant<int, 1>{});
+      else if (ch <= 2)
+        go(std::integral_constant<int, 2>{});
+      else if (ch <= 4)
+        go(std::integral_constant<int, 4>{});
+      else if (ch <= 8)
+        go(std::integral_constant<int, 8>{});
+      else
+        go(std::integral_constant<int, 16>{});
+      launched = true;
+    }
   }
   if (!launched)
     hipLaunchKernelGGL((norm_mod_generic_kernel<Tag, NT, ADD, QNT>), dim3(a.M), dim3(kBlock), 0,
