@@ -901,25 +901,35 @@ bool token_rows(const torch::Tensor& x) {
          reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0;
 }
 
-// A table [1, L, D], [1, L, D/2] or without the leading 1, as the tables op
-// reads it; undefined if it is anything else.
-torch::Tensor table32(const torch::Tensor& t, const torch::Tensor& q) {
-  if (t.scalar_type() != torch::kFloat32 || t.device() != q.device()) return {};
-  const torch::Tensor v = t.dim() == 3 && t.size(0) == 1 ? t.select(0, 0) : t;
+// A [L, D] or [L, D/2] table as the tables op reads it.
+bool table_rows32(const torch::Tensor& t, const torch::Tensor& q) {
   const int64_t L = q.size(1), D = q.size(3);
-  if (v.dim() != 2 || v.size(0) != L || (v.size(1) != D && v.size(1) != D / 2) || v.stride(1) != 1 ||
-      v.stride(0) % 4 != 0 || v.stride(0) < v.size(1) ||
-      reinterpret_cast<uintptr_t>(v.data_ptr()) % 16 != 0)
-    return {};
-  return v;
+  return t.scalar_type() == torch::kFloat32 && t.dim() == 2 && t.size(0) == L &&
+         (t.size(1) == D || t.size(1) == D / 2) && t.stride(1) == 1 && t.stride(0) % 4 == 0 &&
+         t.stride(0) >= t.size(1) && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
 }
 
-bool direct_tables(const torch::Tensor& q, const torch::Tensor& k, torch::Tensor& cos,
-                   torch::Tensor& sin) {
-  if (!token_rows(q) || !token_rows(k) || q.sizes() != k.sizes()) return false;
-  cos = table32(cos, q);
-  sin = table32(sin, q);
-  return cos.defined() && sin.defined() && cos.sizes() == sin.sizes() && cos.strides() == sin.strides();
+// cos and sin on q's device without their leading dims of one.
+void squeeze_tables(torch::Tensor& cos, torch::Tensor& sin, const torch::Tensor& q) {
+  cos = cos.to(q.device());
+  sin = sin.to(q.device());
+  while (cos.dim() > 2) {
+    TORCH_CHECK(cos.size(0) == 1, "freqs_cis cos has non-singleton leading dim: ", cos.sizes());
+    cos = cos.squeeze(0);
+    sin = sin.squeeze(0);
+  }
+}
+
+// Squeezed tables as the paired ops take them: one value a pair, bf16.
+torch::Tensor half_table(const torch::Tensor& t, bool twice) {
+  return (twice ? t.slice(-1, 0, c10::nullopt, 2) : t).contiguous().to(torch::kBFloat16);
+}
+
+// Whether the tables op takes q, k and the squeezed tables where they are.
+bool direct_tables(const torch::Tensor& q, const torch::Tensor& k, const torch::Tensor& cos,
+                   const torch::Tensor& sin) {
+  return token_rows(q) && token_rows(k) && q.sizes() == k.sizes() && table_rows32(cos, q) &&
+         table_rows32(sin, q) && cos.sizes() == sin.sizes() && cos.strides() == sin.strides();
 }
 }  // namespace
 
@@ -986,24 +996,45 @@ torch::Tensor rmsnorm_last(const torch::Tensor& x, const torch::Tensor& weight, 
   return rmsnorm(x.reshape({-1, D}).contiguous(), weight, eps).reshape(x.sizes());
 }
 
-// (q, k) from the tables op where it takes these forms of q, k and the tables
-// and neither q nor k is contiguous (those are rotated in place), else nothing.
-std::vector<torch::Tensor> qk_norm_rope_direct(const torch::Tensor& q, const torch::Tensor& k, double eps,
-                                               const torch::Tensor& q_weight,
-                                               const torch::Tensor& k_weight, torch::Tensor cos,
-                                               torch::Tensor sin) {
-  if (q.is_contiguous() || k.is_contiguous() || !direct_tables(q, k, cos, sin)) return {};
-  auto out = fused_qk_norm_rope_3d_tables(q, k, q.size(1), q.size(2), eps, q_weight, k_weight, cos, sin);
-  return {std::get<0>(out), std::get<1>(out)};
+// q and k [B, L, H, D], both contiguous, in place: the paired op with the
+// tables in the forms that the DiT hands over ([1, L, D], [L, D/2], ...).
+void qk_norm_rope_inplace(torch::Tensor& q, torch::Tensor& k, double eps, torch::Tensor q_weight,
+                          torch::Tensor k_weight, torch::Tensor cos, torch::Tensor sin) {
+  const int64_t B = q.size(0), L = q.size(1), H = q.size(2), D = q.size(3);
+  torch::Tensor q_rows = q.view({B, L * H, D}), k_rows = k.view({B, L * H, D});
+  squeeze_tables(cos, sin, q);
+  const bool twice = cos.size(-1) == D;
+  torch::Tensor c = half_table(cos, twice), s = half_table(sin, twice);
+  fused_qk_norm_rope_3d_paired(q_rows, k_rows, L, H, eps, q_weight, k_weight, c, s);
 }
 
-bool qk_norm_rope_kstage_direct(torch::Tensor& q, torch::Tensor& k, torch::Tensor& k_stage, double eps,
-                                const torch::Tensor& q_weight, const torch::Tensor& k_weight,
-                                torch::Tensor cos, torch::Tensor sin) {
-  if (!direct_tables(q, k, cos, sin)) return false;
-  fused_qk_norm_rope_3d_tables_kstage(q, k, k_stage, q.size(1), q.size(2), eps, q_weight, k_weight, cos,
-                                      sin);
-  return true;
+// New contiguous (q, k) of strided ones: from where they are where the tables
+// op takes these forms, else contiguous copies rotated in place.
+std::tuple<torch::Tensor, torch::Tensor> qk_norm_rope_copies(
+    const torch::Tensor& q, const torch::Tensor& k, double eps, const torch::Tensor& q_weight,
+    const torch::Tensor& k_weight, torch::Tensor cos, torch::Tensor sin) {
+  squeeze_tables(cos, sin, q);
+  if (direct_tables(q, k, cos, sin) && q_weight.dim() == 1 && k_weight.dim() == 1)
+    return fused_qk_norm_rope_3d_tables(q, k, q.size(1), q.size(2), eps, q_weight, k_weight, cos, sin);
+  torch::Tensor qc = q.contiguous(), kc = k.contiguous();
+  qk_norm_rope_inplace(qc, kc, eps, q_weight, k_weight, cos, sin);
+  return {qc, kc};
+}
+
+// The K-stage form: q and k rotated where they are, from fp32 tables where the
+// tables op takes them, else from bf16 copies of their pair values.
+void qk_norm_rope_kstage(torch::Tensor& q, torch::Tensor& k, torch::Tensor& k_stage, double eps,
+                         torch::Tensor q_weight, torch::Tensor k_weight, torch::Tensor cos,
+                         torch::Tensor sin) {
+  const int64_t L = q.size(1), H = q.size(2);
+  squeeze_tables(cos, sin, q);
+  if (direct_tables(q, k, cos, sin)) {
+    fused_qk_norm_rope_3d_tables_kstage(q, k, k_stage, L, H, eps, q_weight, k_weight, cos, sin);
+    return;
+  }
+  const bool twice = cos.size(-1) == q.size(3);
+  torch::Tensor c = half_table(cos, twice), s = half_table(sin, twice);
+  fused_qk_norm_rope_3d_paired_kstage(q, k, k_stage, L, H, eps, q_weight, k_weight, c, s);
 }
 
 }  // namespace joyomni_ops
@@ -1077,11 +1108,14 @@ TORCH_LIBRARY(joyomni_ops, m) {
       "Tensor? beta, Tensor scale, Tensor shift, float eps) -> (Tensor, Tensor)");
   m.def("rmsnorm_last(Tensor x, Tensor weight, float eps, int round_first) -> Tensor");
   m.def(
-      "qk_norm_rope_direct(Tensor q, Tensor k, float eps, Tensor q_weight, Tensor k_weight, "
-      "Tensor cos, Tensor sin) -> Tensor[]");
+      "qk_norm_rope_inplace(Tensor(a!) q, Tensor(b!) k, float eps, Tensor q_weight, "
+      "Tensor k_weight, Tensor cos, Tensor sin) -> ()");
   m.def(
-      "qk_norm_rope_kstage_direct(Tensor(a!) q, Tensor(b!) k, Tensor(c!) k_stage, float eps, "
-      "Tensor q_weight, Tensor k_weight, Tensor cos, Tensor sin) -> bool");
+      "qk_norm_rope_copies(Tensor q, Tensor k, float eps, Tensor q_weight, Tensor k_weight, "
+      "Tensor cos, Tensor sin) -> (Tensor, Tensor)");
+  m.def(
+      "qk_norm_rope_kstage(Tensor(a!) q, Tensor(b!) k, Tensor(c!) k_stage, float eps, "
+      "Tensor q_weight, Tensor k_weight, Tensor cos, Tensor sin) -> ()");
 }
 
 TORCH_LIBRARY_IMPL(joyomni_ops, CUDA, m) {
@@ -1111,6 +1145,7 @@ TORCH_LIBRARY_IMPL(joyomni_ops, CUDA, m) {
   m.impl("layernorm_modulate", &joyomni_ops::layernorm_modulate);
   m.impl("add_gate_layernorm_modulate_fp8", &joyomni_ops::add_gate_layernorm_modulate_fp8);
   m.impl("rmsnorm_last", &joyomni_ops::rmsnorm_last);
-  m.impl("qk_norm_rope_direct", &joyomni_ops::qk_norm_rope_direct);
-  m.impl("qk_norm_rope_kstage_direct", &joyomni_ops::qk_norm_rope_kstage_direct);
+  m.impl("qk_norm_rope_inplace", &joyomni_ops::qk_norm_rope_inplace);
+  m.impl("qk_norm_rope_copies", &joyomni_ops::qk_norm_rope_copies);
+  m.impl("qk_norm_rope_kstage", &joyomni_ops::qk_norm_rope_kstage);
 }

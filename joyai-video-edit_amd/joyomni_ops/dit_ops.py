@@ -50,8 +50,7 @@ from typing import Optional, Sequence, Tuple
 import torch
 
 from . import (fp8_scaled_mm, fused_add_layernorm_scale_shift, fused_qk_norm_rope_3d_grid,
-               fused_qk_norm_rope_3d_paired, fused_qk_norm_rope_3d_paired_kstage, kv_commit_rope,
-               rope_freqs)
+               kv_commit_rope, rope_freqs)
 
 # One dispatch per call: the reshapes, output allocations and launches of these
 # calls are made inside the op (at a few rows they are what a call costs: an
@@ -63,8 +62,9 @@ _fp8_linear = _ops.fp8_linear.default
 _layernorm_modulate = _ops.layernorm_modulate.default
 _add_gate_layernorm_modulate_fp8 = _ops.add_gate_layernorm_modulate_fp8.default
 _rmsnorm_last = _ops.rmsnorm_last.default
-_qk_norm_rope_direct = _ops.qk_norm_rope_direct.default
-_qk_norm_rope_kstage_direct = _ops.qk_norm_rope_kstage_direct.default
+_qk_norm_rope_inplace = _ops.qk_norm_rope_inplace.default
+_qk_norm_rope_copies = _ops.qk_norm_rope_copies.default
+_qk_norm_rope_kstage = _ops.qk_norm_rope_kstage.default
 
 
 def available() -> bool:
@@ -108,44 +108,22 @@ def fused_qk_norm_rope_3d(
     if q.dtype != torch.bfloat16:
         raise RuntimeError(f"fused_qk_norm_rope_3d requires bf16 q/k, got {q.dtype}")
     B, L, H, D = q.shape
-    if not (torch.is_grad_enabled() and (q.requires_grad or k.requires_grad)):
-        # Strided slices and fp32 tables: one pass from where they are
-        # ([1, 3120, 32, 128] of a packed qkv: 50.4 -> 19.3 us on MI355X against
-        # the copies of q and k, the four table kernels and the paired op).
-        out = _qk_norm_rope_direct(q, k, eps, _bf16(q_norm_weight), _bf16(k_norm_weight),
-                                   freqs_cis[0], freqs_cis[1])
-        if out:
-            return out[0], out[1]
-    q = q.contiguous()
-    k = k.contiguous()
-    q_r = q.view(B, L * H, D)
-    k_r = k.view(B, L * H, D)
-    cos_bf16, sin_bf16 = _half_tables_bf16(freqs_cis, L, D, q.device)
-    qw = q_norm_weight.to(torch.bfloat16)
-    kw = k_norm_weight.to(torch.bfloat16)
-    fused_qk_norm_rope_3d_paired(q_r, k_r, L, H, eps, qw, kw, cos_bf16, sin_bf16)
-    return q, k
+    cos, sin = freqs_cis
+    qw, kw = _bf16(q_norm_weight), _bf16(k_norm_weight)
+    if (q.is_contiguous() or k.is_contiguous()
+            or (torch.is_grad_enabled() and (q.requires_grad or k.requires_grad))):
+        q = q.contiguous()  # outside the op: autograd records the copies
+        k = k.contiguous()
+        _qk_norm_rope_inplace(q, k, eps, qw, kw, cos, sin)
+        return q, k
+    # Strided slices and fp32 tables: one pass from where they are
+    # ([1, 3120, 32, 128] of a packed qkv: 50.4 -> 19.3 us on MI355X against
+    # the copies of q and k, the four table kernels and the paired op).
+    return _qk_norm_rope_copies(q, k, eps, qw, kw, cos, sin)
 
 
 def _bf16(w: torch.Tensor) -> torch.Tensor:
     return w if w.dtype is torch.bfloat16 else w.to(torch.bfloat16)
-
-
-def _half_tables_bf16(freqs_cis, L: int, D: int, device):
-    """cos/sin as the paired op takes them: [L, D/2] bf16, from [1, L, D] or
-    [L, D/2] tables, squeezed, halved and cast as sgl_fused_ops.py:80-94 does."""
-    cos, sin = freqs_cis
-    cos = cos.to(device)
-    sin = sin.to(device)
-    while cos.dim() > 2:
-        if cos.shape[0] != 1:
-            raise RuntimeError(f"freqs_cis cos has non-singleton leading dim: {cos.shape}")
-        cos = cos.squeeze(0)
-        sin = sin.squeeze(0)
-    if cos.shape[-1] == D:
-        cos = cos[..., ::2]
-        sin = sin[..., ::2]
-    return cos.contiguous().to(torch.bfloat16), sin.contiguous().to(torch.bfloat16)
 
 
 def fused_qk_norm_rope_3d_kstage(
@@ -176,16 +154,9 @@ def fused_qk_norm_rope_3d_kstage(
     B, L, H, D = q.shape
     if k_stage is None:
         k_stage = torch.empty((B, L, H, D), dtype=torch.bfloat16, device=q.device)
-    if not (torch.is_grad_enabled() and (q.requires_grad or k.requires_grad)):
-        # fp32 tables are read as they are
-        if _qk_norm_rope_kstage_direct(q, k, k_stage, eps, _bf16(q_norm_weight).contiguous(),
-                                       _bf16(k_norm_weight).contiguous(), freqs_cis[0],
-                                       freqs_cis[1]):
-            return q, k, k_stage
-    cos, sin = _half_tables_bf16(freqs_cis, L, D, q.device)
-    fused_qk_norm_rope_3d_paired_kstage(q, k, k_stage, L, H, eps,
-                                        q_norm_weight.to(torch.bfloat16).contiguous(),
-                                        k_norm_weight.to(torch.bfloat16).contiguous(), cos, sin)
+    cos, sin = freqs_cis
+    _qk_norm_rope_kstage(q, k, k_stage, eps, _bf16(q_norm_weight).contiguous(),
+                         _bf16(k_norm_weight).contiguous(), cos, sin)
     return q, k, k_stage
 
 

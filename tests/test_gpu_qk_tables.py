@@ -131,3 +131,36 @@ def test_captured_pass_replays(dev):
         graph.replay()
         torch.cuda.synchronize()
         assert all(torch.equal(a, b) for a, b in zip(out, want))
+
+
+@pytest.mark.parametrize("form", ["sin_with_a_leading_dim", "sin_squeezed_once_too_often",
+                                  "weight_of_rank_2"])
+def test_forms_that_the_paired_op_refuses(dev, form):
+    """sin loses a leading dim only where cos does, as the reference's caller squeezes them, and
+    the weights are 1D."""
+    from joyomni_ops import dit_ops
+    L = 1 if form == "sin_squeezed_once_too_often" else 5
+    qkv, qw, kw, cos, sin = _inputs(dev, 2, L, 4, 64, True)
+    if form == "sin_with_a_leading_dim":
+        sin = sin.unsqueeze(0)
+    elif form == "sin_squeezed_once_too_often":
+        cos = cos.unsqueeze(0)
+    else:
+        qw = qw.unsqueeze(0)
+    with pytest.raises(RuntimeError):
+        dit_ops.fused_qk_norm_rope_3d(qkv[:, :, 0], qkv[:, :, 1], qw, kw, (cos, sin))
+
+
+@pytest.mark.parametrize("kstage", [False, True])
+@pytest.mark.parametrize("tables", ["host", "bf16_rank4"])
+def test_tables_that_are_converted_first(dev, tables, kstage):
+    import joyomni_ops as jo
+    from joyomni_ops import dit_ops
+    qkv, qw, kw, cos, sin = _inputs(dev, 1, 9, 8, 128, True)
+    q, k = qkv[:, :, 0], qkv[:, :, 1]
+    want = _general(jo, q, k, qw, kw, cos, sin)
+    given = ((cos.cpu(), sin.cpu()) if tables == "host" else
+             (cos.to(torch.bfloat16)[None, None], sin.to(torch.bfloat16)[None, None]))
+    call = dit_ops.fused_qk_norm_rope_3d_kstage if kstage else dit_ops.fused_qk_norm_rope_3d
+    got = call(q, k, qw, kw, given)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
