@@ -67,6 +67,29 @@ _qk_norm_rope_copies = _ops.qk_norm_rope_copies.default
 _qk_norm_rope_kstage = _ops.qk_norm_rope_kstage.default
 
 
+# Shapes of the results, for tracing (torch.compile and fake tensors), of the ops
+# that allocate outputs whose calls traced when the Python shims allocated them;
+# the ops that only write into their arguments need none.
+@torch.library.register_fake("joyomni_ops::quantize_activation")
+@torch.library.register_fake("joyomni_ops::gelu_quantize_activation")
+def _(x):
+    K = x.shape[-1]
+    M = x.numel() // K
+    return x.new_empty((M, K), dtype=torch.float8_e4m3fn), x.new_empty((M, 1), dtype=torch.float32)
+
+
+@torch.library.register_fake("joyomni_ops::add_gate_layernorm_modulate_fp8")
+def _(x, residual, gate, gamma, beta, scale, shift, eps):
+    B, L, D = x.shape
+    return (x.new_empty((B * L, D), dtype=torch.float8_e4m3fn),
+            x.new_empty((B * L, 1), dtype=torch.float32))
+
+
+@torch.library.register_fake("joyomni_ops::qk_norm_rope_copies")
+def _(q, k, eps, q_weight, k_weight, cos, sin):
+    return q.new_empty(q.shape), k.new_empty(k.shape)
+
+
 def available() -> bool:
     """The reference's availability probe (sgl_fused_ops.py:14-27): the ops load at import."""
     return True
