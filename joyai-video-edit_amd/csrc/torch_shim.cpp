@@ -1149,3 +1149,14 @@ TORCH_LIBRARY_IMPL(joyomni_ops, CUDA, m) {
   m.impl("qk_norm_rope_copies", &joyomni_ops::qk_norm_rope_copies);
   m.impl("qk_norm_rope_kstage", &joyomni_ops::qk_norm_rope_kstage);
 }
+
+// Ops that allocate results which autograd never saw: the ops that they call
+// write into their arguments, so no result claims a gradient that nothing
+// computes. (Ops with results of their own, such as rmsnorm_last, keep the
+// dispatcher's default: a result that warns when it is differentiated.)
+TORCH_LIBRARY_IMPL(joyomni_ops, Autograd, m) {
+  m.impl("quantize_activation", torch::CppFunction::makeFallthrough());
+  m.impl("gelu_quantize_activation", torch::CppFunction::makeFallthrough());
+  m.impl("add_gate_layernorm_modulate_fp8", torch::CppFunction::makeFallthrough());
+  m.impl("qk_norm_rope_copies", torch::CppFunction::makeFallthrough());
+}

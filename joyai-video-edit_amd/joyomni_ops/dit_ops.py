@@ -366,6 +366,8 @@ def fp8_linear(x: torch.Tensor, weight_fp8: torch.Tensor, weight_scale: torch.Te
                bias: Optional[torch.Tensor] = None, out_dtype=torch.bfloat16) -> torch.Tensor:
     """Fp8Linear.forward (fp8_linear.py:155-169): x [..., K] bf16 -> per-token
     fp8 + scales -> fp8_scaled_mm with the per-channel weight scales and bias."""
+    if x.requires_grad:
+        x = x.detach()  # its quantized form carries no gradient
     return _fp8_linear(x, weight_fp8, weight_scale, bias, out_dtype)
 
 

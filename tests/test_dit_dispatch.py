@@ -113,3 +113,27 @@ def test_compiled_without_a_graph_break(dev, name):
         got = torch.compile(fn, backend="aot_eager", fullgraph=True)(*copy(args))
         for a, b in zip(got, want):
             assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,grad_on", [(n, "x") for n in TRACED + ["fp8_linear"]] +
+                         [(n, "vector") for n in TRACED[2:] + ["fp8_linear"]])
+def test_results_claim_no_gradient(dev, name, grad_on):
+    """What these calls write through quantized or in-place results has no gradient, whatever
+    the inputs ask for; q and k rotated in place keep the history of what they were, and an
+    Fp8Linear's output that of its bias."""
+    from joyomni_ops import dit_ops
+    new = lambda *s, dt=torch.bfloat16: torch.ones(*s, dtype=dt, device=dev)  # noqa: E731
+    if name == "fp8_linear":
+        args = (new(2, 8, 256), new(64, 256).to(torch.float8_e4m3fn).t(),
+                new(64, dt=torch.float32), new(64))
+        fn, wanted = dit_ops.fp8_linear, args[0] if grad_on == "x" else args[3]
+    else:
+        fn, args = _calls(dit_ops, new)[name]
+        wanted = args[{"x": 1 if name == "add_norm_fp8" else 0, "vector": 2}[grad_on]]
+    out = fn(*(a.requires_grad_() if a is wanted else a for a in args))
+    flags = [t.requires_grad for t in (out if isinstance(out, tuple) else (out,))]
+    if grad_on == "x" and name.startswith("qk_rope"):
+        assert flags == [True, False, False][:len(flags)]
+    else:
+        assert flags == [name == "fp8_linear" and grad_on == "vector"] * len(flags)
