@@ -1263,15 +1263,18 @@ int auto_shape(int cus, int M, int N) {
 constexpr int64_t kSplitCap = int64_t{1} << 30;  // largest partial buffer a split uses
 
 // Estimated time of the streaming kernel, ns: the launch, first loads and last
-// exchange; every row of A once a workgroup out of L2 (109 KB/us a CU); and B
-// at what HBM gives all CUs (5.0 TB/s) or a CU can draw (33 KB/us). Fitted to
-// M = 1, 16, 40 and 77 at N = 4096 to 16384, mostly within 15% of what was
-// measured.
-int64_t stream_ns(int cus, int M, int N, int K, int nb) {
-  const int64_t tiles = (N + nb * 16 - 1) / (nb * 16), rounds = (tiles + cus - 1) / cus;
-  const int64_t a = rounds * ((M + 15) / 16 * 16) * K / 109;
-  const int64_t b = static_cast<int64_t>(N) * K / 5000, b_cu = rounds * nb * 16 * K / 33;
-  return 3000 + a + (b > b_cu ? b : b_cu);
+// exchange; the busiest CU's rows of A (70 KB/us) and columns of B (35 KB/us),
+// or B at what HBM gives all CUs (5.3 TB/s) with A beside it, whichever is
+// longer; and what a workgroup and a block of the exchange cost. The constants
+// here and in plan_gemm were fitted so that no choice was slower than the
+// kernel it replaces on 770 shapes (1 to 80 rows, N 512 to 16384, K 512 to
+// 16384), with weights from HBM and with cached ones: each of the four widths
+// measured on each, 0.91 of the time that the best choice saves is saved.
+int64_t stream_ns(int M, int N, int K, int nb) {
+  const int64_t tiles = (N + nb * 16 - 1) / (nb * 16);  // at most one a CU
+  const int64_t mb = (M + 15) / 16, a = mb * 16 * K, b = static_cast<int64_t>(nb) * 16 * K;
+  const int64_t cu = a / 70 + b / 35, hbm = static_cast<int64_t>(N) * K / 5300 + a / 85;
+  return 3000 + (cu > hbm ? cu : hbm) + 2 * tiles + 40 * mb * nb;
 }
 
 struct GemmPlan {
@@ -1337,22 +1340,24 @@ GemmPlan plan_gemm(const GemmArgs& g, int64_t ws_bytes) {
   const bool splits = best >= 0 && best * 20 < unsplit * 17;
   if (splits) p = split;
   // Few rows: the streaming kernel where it is estimated faster than the
-  // choice so far, which takes 3 us and its operand bytes at 49 KB/us a CU; with
-  // a split, 4 us more for the second launch, and 75 KB/us where workgroups
-  // share a CU.
+  // choice so far: 3.6 us and its operand bytes at 52 KB/us a CU (3 us more for
+  // the two waves of 64x96 tiles); with a split 10.5 us for the two launches and
+  // 100 KB/us, or 30 where workgroups share a CU (streaming was faster on every
+  // such shape). A weight that comes from HBM decides most of them: 80x2048x6144
+  // 10.6 us split in four, 12.3 streamed (cached 9.5 and 7.1). Only where one
+  // round of workgroups takes all columns: past that the short K's measured up
+  // to half slower (57x17632x128 5.1 -> 7.6).
   if (g.M <= kStreamRows) {
-    int64_t other = 3000 + unsplit / 49;
+    int64_t other = 3600 + unsplit / 52 + (p.shape == 11 ? 3000 : 0);
     if (splits) {
       const int64_t t = split.shape == 5 ? 128 : 64;
       const int64_t wgs = (g.M + t - 1) / t * ((g.N + t - 1) / t) * split.splits, per = (wgs + cus - 1) / cus;
-      other = 7000 + per * 2 * t * (g.K / split.splits) / (per > 1 ? 75 : 49);
+      other = 10500 + per * 2 * t * (g.K / split.splits) / (per > 1 ? 30 : 100);
     }
     for (int nb = 1; nb <= 4; ++nb) {
-      const int64_t ns = stream_ns(cus, g.M, g.N, g.K, nb);
-      // On a tie up to 32 rows take the wider tile (fewer workgroups' fixed
-      // cost: 1x12288x4096 12.1 / 10.3 us with three column blocks, 11.7 / 9.9
-      // with four), above the narrower one (at 77 rows 16.9 / 12.5 and 17.8 / 12.6).
-      if (ns < other || (ns == other && p.shape >= kStream && g.M <= 32)) {
+      if (g.N > cus * nb * 16) continue;
+      const int64_t ns = stream_ns(g.M, g.N, g.K, nb);
+      if (ns < other) {
         other = ns;
         p = GemmPlan{kStream + nb * 16, 1};
       }

@@ -219,6 +219,17 @@ def test_gemm_workspace_bytes(abi):
         lib.jo_set_launch_override(abi.JO_KNOB_GEMM_SPLIT, -1)
 
 
+def test_gemm_few_rows_split_where_that_is_faster(abi):
+    """Few rows and a long K with few columns: the split K (a workspace) where the streaming
+    kernel, which takes none, measured slower with weights from HBM."""
+    wb = abi.lib().jo_fp8_scaled_mm_workspace_bytes
+    for M, N, K, splits in [(48, 1024, 11776, 4), (65, 1536, 6144, 4), (80, 2048, 6144, 4),
+                            (80, 4096, 11776, 2)]:
+        assert wb(M, N, K) == splits * M * N * 4, (M, N, K)
+    for M, N, K in [(1, 4096, 4096), (16, 2048, 11776), (48, 4096, 4096), (77, 12288, 4096)]:
+        assert wb(M, N, K) == 0, (M, N, K)
+
+
 def test_launch_override_env_values_are_checked(tmp_path):
     """An environment override the knob does not accept is ignored with a
     message (a fresh process, since the variables are read at load)."""
