@@ -1200,7 +1200,7 @@ int cu_count() {
 
 // Launch shapes. kPair + rows: the eight-wave pair kernel with tiles of that
 // many rows x 256 columns (a multiple of 16 from 96 to 256); 2: the
-// register-staged kernel; 5, 6, 8, 10, 11: the small-tile kernel.
+// register-staged kernel; 5, 6, 8, 10, 11, 12: the small-tile kernel.
 // kStream + 16 NB: the streaming kernel with NB column blocks.
 constexpr int kPair = 1000;
 constexpr int kStream = 2000;
@@ -1213,9 +1213,17 @@ constexpr int kStream = 2000;
 // higher, by the 32 KB of B a stage that they wait on when the weight comes
 // from HBM ([256, 16384] x 4096 in a whole MLP: 96-row tiles 4 us slower than
 // the 128x128 ones, though level with cached weights).
-int64_t pair_cost(int cus, int M, int N, int rows) {
+// Up to 128 rows in one row of tiles and a long K: no two workgroups share B
+// then, and a CU draws its 32 KB a stage from HBM in the time of 23,500, so 128x192
+// tiles are faster where they fit one round (us, weights from HBM, 96- or
+// 112-row tiles / 128x192: 74x39720x3840 36.2 / 33.4, 101x35392x4096 41.2 / 39.6;
+// with K up to 1280 the pair kernel is: 71x32912x1024 12.3 / 13.2).
+bool one_row(int M, int K) { return M <= 128 && K > 1280; }
+
+int64_t pair_cost(int cus, int M, int N, int K, int rows) {
   const int64_t tiles = static_cast<int64_t>((M + rows - 1) / rows) * ((N + 255) / 256);
-  const int64_t stage = 96 * rows + 800 > 56 * rows + 8500 ? 96 * rows + 800 : 56 * rows + 8500;
+  int64_t stage = 96 * rows + 800 > 56 * rows + 8500 ? 96 * rows + 800 : 56 * rows + 8500;
+  if (one_row(M, K) && M <= rows && stage < 23500) stage = 23500;
   return (tiles + cus - 1) / cus * stage / 50;
 }
 
@@ -1238,19 +1246,20 @@ int64_t small_cost(int cus, int M, int N, int bm, int bn) {
 // x 16384 118 -> 101 (112), [512, 12288] x 4096 30.6 -> 25.7 (128); the
 // small tiles at M = 256: [256, 4096] x 4096 34.2 -> 11.4 us (64x64),
 // [256, 12288] x 4096 42.4 -> 22.0 us (128x96).
-int auto_shape(int cus, int M, int N) {
+int auto_shape(int cus, int M, int N, int K) {
   int shape = 0;
   int64_t best = INT64_MAX;
   for (int rows = 256; rows >= 96; rows -= 16) {
-    const int64_t c = pair_cost(cus, M, N, rows);
+    const int64_t c = pair_cost(cus, M, N, K, rows);
     if (c < best) {
       best = c;
       shape = kPair + rows;
     }
   }
   // Larger tiles first: a tie goes to the smaller one.
-  const int small[5][3] = {{5, 128, 128}, {10, 128, 96}, {8, 64, 128}, {11, 64, 96}, {6, 64, 64}};
+  const int small[6][3] = {{12, 128, 192}, {5, 128, 128}, {10, 128, 96}, {8, 64, 128}, {11, 64, 96}, {6, 64, 64}};
   for (const auto& t : small) {
+    if (t[0] == 12 && !one_row(M, K)) continue;
     const int64_t c = small_cost(cus, M, N, t[1], t[2]);
     if (c <= best) {
       best = c;
@@ -1298,14 +1307,15 @@ int64_t split_bytes(int M, int N, int splits) {
   return splits > 1 ? static_cast<int64_t>(splits) * M * N * 4 : 0;
 }
 
-int64_t shape_cost(int cus, int shape, int M, int N) {
+int64_t shape_cost(int cus, int shape, int M, int N, int K) {
   switch (shape) {
     case 5: return small_cost(cus, M, N, 128, 128);
     case 6: return small_cost(cus, M, N, 64, 64);
     case 8: return small_cost(cus, M, N, 64, 128);
     case 10: return small_cost(cus, M, N, 128, 96);
     case 11: return small_cost(cus, M, N, 64, 96);
-    default: return pair_cost(cus, M, N, shape - kPair);
+    case 12: return small_cost(cus, M, N, 128, 192);
+    default: return pair_cost(cus, M, N, K, shape - kPair);
   }
 }
 
@@ -1326,7 +1336,7 @@ GemmPlan plan_gemm(const GemmArgs& g, int64_t ws_bytes) {
   const int forced = launch_knob(JO_KNOB_GEMM_SHAPE);
   const int fsplit = launch_knob(JO_KNOB_GEMM_SPLIT);
   const int cus = cu_count();
-  GemmPlan p{forced >= 0 ? knob_shape(forced) : auto_shape(cus, g.M, g.N), 1};
+  GemmPlan p{forced >= 0 ? knob_shape(forced) : auto_shape(cus, g.M, g.N, g.K), 1};
   const int64_t room = ws_bytes < kSplitCap ? ws_bytes : kSplitCap;
   auto split_ok = [&](int sp) {
     return g.K > 0 && g.K % (kQBK * sp) == 0 && split_bytes(g.M, g.N, sp) <= room;
@@ -1336,7 +1346,7 @@ GemmPlan plan_gemm(const GemmArgs& g, int64_t ws_bytes) {
     return p;
   }
   if (forced >= 0) return p;
-  const int64_t unsplit = shape_cost(cus, p.shape, g.M, g.N) * g.K;
+  const int64_t unsplit = shape_cost(cus, p.shape, g.M, g.N, g.K) * g.K;
   int64_t best = -1;
   GemmPlan split{p.shape, 1};
   const int cand[2][3] = {{5, 128, 128}, {6, 64, 64}};
@@ -1401,6 +1411,8 @@ int launch_gemm(const GemmArgs& g, hipStream_t stream, int64_t ws_bytes) {
     launch_small<OutTag, 128, 96, 4, 4, 4>(g, stream);
   else if (shape == 11)
     launch_small<OutTag, 64, 96, 2, 4, 2>(g, stream);
+  else if (shape == 12)
+    launch_small<OutTag, 128, 192, 4, 3>(g, stream);
   else if (shape < kStream)
     launch_pair_rows<OutTag>(g, stream, shape - kPair);
   else

@@ -28,3 +28,13 @@ def test_tile_heights(dev, rows, K, dtype):
                   set(range(rows)) | set(range(M - 32, M)))
     idx = torch.tensor(pick)
     check(out[idx.to(dev)], a, w.t(), sa, sb, bias, f"[{M},{N},{K}] {rows}-row tiles", rows=idx)
+
+
+@pytest.mark.parametrize("M,N,K", [(128, 32776, 1296), (70, 40960, 1408)])
+def test_one_row_of_wide_tiles(dev, M, N, K):
+    """128x192 tiles: up to 128 rows, a long K and more columns than 128 of them a CU cover."""
+    import joyomni_ops as jo
+    a, w, sa, sb, bias = operands(M, N, K, M + K)
+    out = jo.fp8_scaled_mm(a.to(dev), w.to(dev).t(), sa.to(dev), sb.to(dev), torch.bfloat16,
+                           bias.to(dev))
+    check(out, a, w.t(), sa, sb, bias, f"[{M},{N},{K}]")
