@@ -1,6 +1,6 @@
 """The fused norms at row lengths that are a multiple of 4 but not of 8 (16-bit types): the
 edges of each thread's chunk count (1, 2, 4, 8 and 16 chunks of four over 256 threads) and
-the first length past them (the element-wise kernel), through the oracle comparisons of
+lengths on either side of them (the element-wise kernel), through the oracle comparisons of
 test_gpu_norms and test_gpu_norm_quant; and rows of a length that is a multiple of 8 whose
 stride is only a multiple of 4."""
 from __future__ import annotations
@@ -15,7 +15,7 @@ from oracle import ops
 
 pytestmark = pytest.mark.gpu
 
-LENGTHS = [4, 1020, 1028, 2044, 2052, 4092, 4100, 8188, 8196, 16380, 16388]
+LENGTHS = [4, 252, 260, 1020, 1028, 2044, 2052, 4092, 4100, 8188, 8196, 16380, 16388]
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
