@@ -32,7 +32,7 @@
 extern "C" {
 #endif
 
-#define JO_ABI_VERSION 4
+#define JO_ABI_VERSION 5
 
 /* Status codes. */
 #define JO_OK 0
@@ -58,7 +58,9 @@ const char* jo_last_error(void);
 int jo_abi_version(void);
 
 /* Launch-shape knobs. Each selects how a kernel is spread over waves, never
- * what it computes: results are identical under every setting. The value is
+ * what it computes: results are identical under every setting of the QK and KV
+ * knobs, and under those of the GEMM up to the order in which the fp32 products
+ * of a row are added. The value is
  * -1 (the library's own choice) unless the environment variable named below
  * was set when the library was loaded, or jo_set_launch_override() changed it.
  *   JO_KNOB_QK_SPLIT    waves per token of the QK norm + RoPE kernels: 1, 2,
@@ -76,7 +78,9 @@ int jo_abi_version(void);
  *                       tile, taken by the 128x128 and 64x64 tiles when
  *                       jo_fp8_scaled_mm_ws has the workspace for it and
  *                       K % (128 x split) == 0 (env JO_GEMM_SPLIT)
- * No reference counterpart (tuning and test hook). */
+ * No reference counterpart (tuning and test hook). Up to version 4 the GEMM
+ * shapes 1, 4, 7 and 9 were 256x128, 224x128, 128x256 on a small tile's kernel
+ * and 128x192, which this library no longer takes as overrides. */
 #define JO_KNOB_QK_SPLIT 0
 #define JO_KNOB_KV_SPLIT 1
 #define JO_KNOB_GEMM_SHAPE 2

@@ -20,8 +20,9 @@ int launch_status(const char* op);
 
 // Launch-shape override of a JO_KNOB_* knob: -1 (automatic choice) unless the
 // environment set it when the library was loaded (JO_QK_SPLIT, JO_KV_SPLIT,
-// JO_GEMM_SHAPE) or jo_set_launch_override() changed it since. Results never
-// depend on a knob, only the launch shape does.
+// JO_GEMM_SHAPE, JO_GEMM_SPLIT) or jo_set_launch_override() changed it since.
+// Results do not depend on the QK and KV knobs; on the GEMM's only in the order
+// of its fp32 sums.
 int launch_knob(int knob);
 
 #define JO_REQUIRE(cond, ...)      \

@@ -14,7 +14,7 @@ thread_local char g_last_error[512] = {0};
 constexpr int kKnobs = 4;
 
 // The values each knob accepts besides -1 (the library's own choice):
-// QK waves per token 1, 2, 4, 6, 8; KV rows on 1 or 2 waves; GEMM shapes 0-9;
+// QK waves per token 1, 2, 4, 6, 8; KV rows on 1 or 2 waves; GEMM shapes 0-11;
 // GEMM K splits 1, 2, 4, 8.
 bool knob_value_ok(int knob, int v) {
   if (v == -1) return true;

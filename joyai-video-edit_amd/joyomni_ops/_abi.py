@@ -16,7 +16,7 @@ LIB_NAME = "libjoyomni_hip.so"
 
 # The header's JO_ABI_VERSION this binding's SIGNATURES follow; a library
 # reporting another version is refused at load.
-JO_ABI_VERSION = 4
+JO_ABI_VERSION = 5
 
 JO_OK = 0
 JO_ERR_INVALID = 1

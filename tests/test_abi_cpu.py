@@ -58,7 +58,7 @@ def test_ctypes_signatures_match_header(abi):
 
 
 def test_abi_version(abi):
-    assert abi.lib().jo_abi_version() == 4
+    assert abi.lib().jo_abi_version() == 5
 
 
 # Launch-size bounds of the entry points (work items of one launch < 2^32).
