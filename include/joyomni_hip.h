@@ -440,6 +440,18 @@ int jo_fp8_scaled_mm_ws(const void* mat_a, int64_t lda, const void* mat_b, int64
  * split K (then no workspace is needed). A host-side computation. */
 int64_t jo_fp8_scaled_mm_workspace_bytes(int64_t M, int64_t N, int64_t K);
 
+/* The launch that jo_fp8_scaled_mm_ws makes of an [M, K] x [K, N] product with
+ * the workspace it asks for, 16-byte aligned scales and bias and rows K bytes
+ * apart, under the current launch knobs and on the current device's CUs:
+ * plan[0] = JO_GEMM_*, plan[1] x plan[2] = rows x columns of a workgroup's tile,
+ * plan[3] = workgroups that share a tile's K. A host-side computation, for tests
+ * and tuning; no reference counterpart. */
+#define JO_GEMM_STAGED 0 /* register-staged */
+#define JO_GEMM_PAIR 1   /* eight waves, 256 columns, 96 to 256 rows */
+#define JO_GEMM_SMALL 2  /* small tiles, the only kernel that splits K */
+#define JO_GEMM_STREAM 3 /* up to 80 rows in one tile row, K over the waves */
+int jo_fp8_scaled_mm_plan(int64_t M, int64_t N, int64_t K, int32_t* plan);
+
 /* jo_fp8_scaled_mm_ws without a caller workspace, for callers that cannot
  * allocate (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc): no counterpart in the reference. The split-K partials

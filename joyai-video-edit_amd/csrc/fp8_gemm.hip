@@ -1517,6 +1517,34 @@ extern "C" int64_t jo_fp8_scaled_mm_workspace_bytes(int64_t M, int64_t N, int64_
   return split_bytes(g.M, g.N, p.splits);
 }
 
+extern "C" int jo_fp8_scaled_mm_plan(int64_t M, int64_t N, int64_t K, int32_t* plan) {
+  JO_REQUIRE(M > 0 && N > 0 && K > 0 && M <= INT32_MAX && N <= INT32_MAX && K <= INT32_MAX,
+             "fp8_scaled_mm_plan: bad shape");
+  JO_REQUIRE(plan != nullptr, "fp8_scaled_mm_plan: null pointer");
+  GemmArgs g{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, K, K, N,
+             static_cast<int>(M), static_cast<int>(N), static_cast<int>(K)};
+  const GemmPlan p = plan_gemm(g, kSplitCap);
+  int kernel = JO_GEMM_SMALL, rows = 0, cols = 0;
+  switch (p.shape) {
+    case 2: kernel = JO_GEMM_STAGED; rows = kBM; cols = kBN; break;
+    case 5: rows = 128; cols = 128; break;
+    case 6: rows = 64; cols = 64; break;
+    case 8: rows = 64; cols = 128; break;
+    case 10: rows = 128; cols = 96; break;
+    case 11: rows = 64; cols = 96; break;
+    case 12: rows = 128; cols = 192; break;
+    default:
+      if (p.shape < kStream) {
+        kernel = JO_GEMM_PAIR; rows = p.shape - kPair; cols = 256;
+      } else {
+        kernel = JO_GEMM_STREAM; rows = (g.M + 15) / 16 * 16; cols = p.shape - kStream;
+      }
+  }
+  const int32_t found[4] = {kernel, rows, cols, p.splits};
+  for (int i = 0; i < 4; ++i) plan[i] = found[i];
+  return JO_OK;
+}
+
 extern "C" int jo_fp8_scaled_mm_noalloc(const void* mat_a, int64_t lda, const void* mat_b,
                                         int64_t ldb, const float* scales_a,
                                         const float* scales_b, const void* bias, void* out,

@@ -35,6 +35,11 @@ JO_KNOB_KV_SPLIT = 1
 JO_KNOB_GEMM_SHAPE = 2
 JO_KNOB_GEMM_SPLIT = 3
 
+JO_GEMM_STAGED = 0
+JO_GEMM_PAIR = 1
+JO_GEMM_SMALL = 2
+JO_GEMM_STREAM = 3
+
 _P = c_void_p
 _I64 = c_int64
 _F = c_float
@@ -81,6 +86,7 @@ SIGNATURES: dict[str, list] = {
     "jo_fp8_scaled_mm_ws": [_P, _I64, _P, _I64, _P, _P, _P, _P, _I64, _I64, _I64, _I64, c_int, _P,
                             _I64, _P],
     "jo_fp8_scaled_mm_workspace_bytes": [_I64, _I64, _I64],
+    "jo_fp8_scaled_mm_plan": [_I64, _I64, _I64, _P],
     "jo_fp8_scaled_mm_noalloc": [_P, _I64, _P, _I64, _P, _P, _P, _P, _I64, _I64, _I64, _I64, c_int,
                                  _P],
     "jo_kv_commit_rope": [
@@ -126,6 +132,13 @@ def lib() -> ctypes.CDLL:
         fn.argtypes = argtypes
     _lib = handle
     return _lib
+
+
+def gemm_plan(M: int, N: int, K: int) -> tuple[int, int, int, int]:
+    """(JO_GEMM_* kernel, tile rows, tile columns, K split) of jo_fp8_scaled_mm_plan."""
+    plan = (c_int32 * 4)()
+    call("jo_fp8_scaled_mm_plan", M, N, K, plan)
+    return tuple(plan)
 
 
 def last_error() -> str:

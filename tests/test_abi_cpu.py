@@ -219,6 +219,33 @@ def test_gemm_workspace_bytes(abi):
         lib.jo_set_launch_override(abi.JO_KNOB_GEMM_SPLIT, -1)
 
 
+@pytest.mark.parametrize("M,N,K,plan", [
+    (3120, 12288, 4096, ("PAIR", 208, 256, 1)), (3120, 4096, 16384, ("PAIR", 208, 256, 1)),
+    (256, 12288, 4096, ("SMALL", 128, 96, 1)), (256, 4096, 16384, ("SMALL", 128, 128, 4)),
+    (64, 4096, 16384, ("SMALL", 64, 64, 4)), (120, 40960, 4096, ("SMALL", 128, 192, 1)),
+    (77, 12288, 4096, ("STREAM", 80, 48, 1)), (1, 8, 16, ("STREAM", 16, 16, 1)),
+    (80, 8192, 8192, ("SMALL", 64, 64, 1)), (16, 16392, 128, ("SMALL", 64, 96, 1))])
+def test_gemm_plan(abi, M, N, K, plan):
+    """The kernel, tile and split of the default choice (256 CUs)."""
+    assert abi.gemm_plan(M, N, K) == (getattr(abi, "JO_GEMM_" + plan[0]), *plan[1:])
+
+
+def test_gemm_plan_of_overrides_and_bad_shapes(abi):
+    lib = abi.lib()
+    try:
+        for v, tile in {0: (256, 256), 1: (208, 256), 2: (256, 256), 3: (224, 256),
+                        4: (160, 256), 5: (128, 128), 6: (64, 64), 7: (128, 256), 8: (64, 128),
+                        9: (112, 256), 10: (128, 96), 11: (64, 96)}.items():
+            lib.jo_set_launch_override(abi.JO_KNOB_GEMM_SHAPE, v)
+            kernel = (abi.JO_GEMM_STAGED if v == 2 else abi.JO_GEMM_PAIR if tile[1] == 256 else
+                      abi.JO_GEMM_SMALL)
+            assert abi.gemm_plan(500, 520, 256) == (kernel, *tile, 1)
+    finally:
+        lib.jo_set_launch_override(abi.JO_KNOB_GEMM_SHAPE, -1)
+    assert lib.jo_fp8_scaled_mm_plan(0, 8, 16, None) == abi.JO_ERR_INVALID
+    assert lib.jo_fp8_scaled_mm_plan(1, 8, 16, None) == abi.JO_ERR_INVALID
+
+
 def test_gemm_few_rows_split_where_that_is_faster(abi):
     """Few rows and a long K with few columns: the split K (a workspace) where the streaming
     kernel, which takes none, measured slower with weights from HBM."""

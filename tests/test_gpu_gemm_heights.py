@@ -19,7 +19,9 @@ pytestmark = pytest.mark.gpu
                                      (640, torch.bfloat16)])
 def test_tile_heights(dev, rows, K, dtype):
     import joyomni_ops as jo
+    from joyomni_ops import _abi
     M, N = 16 * rows - 5, 4096 - 8
+    assert _abi.gemm_plan(M, N, K) == (_abi.JO_GEMM_PAIR, rows, 256, 1)
     a, w, sa, sb, bias = operands(M, N, K, rows + K, dtype)
     out = jo.fp8_scaled_mm(a.to(dev), w.to(dev).t(), sa.to(dev), sb.to(dev), dtype, bias.to(dev))
     # The first tile, the rows around each wave row's and tile's edge, and the ragged last tile.
@@ -34,6 +36,8 @@ def test_tile_heights(dev, rows, K, dtype):
 def test_one_row_of_wide_tiles(dev, M, N, K):
     """128x192 tiles: up to 128 rows, a long K and more columns than 128 of them a CU cover."""
     import joyomni_ops as jo
+    from joyomni_ops import _abi
+    assert _abi.gemm_plan(M, N, K) == (_abi.JO_GEMM_SMALL, 128, 192, 1)
     a, w, sa, sb, bias = operands(M, N, K, M + K)
     out = jo.fp8_scaled_mm(a.to(dev), w.to(dev).t(), sa.to(dev), sb.to(dev), torch.bfloat16,
                            bias.to(dev))
