@@ -21,11 +21,10 @@ pytestmark = pytest.mark.gpu
 @pytest.fixture(params=["auto", "0", "1", "2", "3", "4", "5", "6", "7", "8", "9", "10", "11"],
                 autouse=True)
 def gemm_shape(request):
-    """Every kernel variant: the default choice, 256x256 (8 waves), 256x128
-    (4 waves), the register-staged kernel (also the K % 64 != 0 path), 224x256
-    (8 waves, 4 and 3 row blocks), 224x128 (4 waves), and the small-tile
-    kernel at 128x128, 64x64, 64x128, 128x192 and 128x96 (4 waves), 128x256
-    (8 waves) and 64x96 (2 waves)."""
+    """The default choice and every override: the eight-wave kernel at 256, 208,
+    224, 160, 128 and 112 rows x 256 columns (0, 1, 3, 4, 7, 9), the
+    register-staged kernel (2), and the small-tile kernel at 128x128, 64x64,
+    64x128 and 128x96 (four waves: 5, 6, 8, 10) and 64x96 (two: 11)."""
     from joyomni_ops import _abi
     value = -1 if request.param == "auto" else int(request.param)
     _abi.call("jo_set_launch_override", _abi.JO_KNOB_GEMM_SHAPE, value)
@@ -150,9 +149,10 @@ _TEXT_ORACLE = {}
 def test_fp8_scaled_mm_text_stream_shapes(dev, M, N, K):
     """The text stream's Fp8Linear shapes (a few hundred prompt tokens against
     the hidden 4096 / MLP 16384 weights), where the automatic choice takes the
-    small-tile kernel (64x64, 128x128, 64x96 and 128x96 on the qkv projection's
-    12288 columns with a ragged last row of tiles, or, at 512 x 16384, 128x256);
-    every output against the exact oracle (computed once per shape, reused
+    streaming kernel (77 rows), the small-tile kernel (64x96 and 128x96 on the
+    qkv projection's 12288 columns with a ragged last row of tiles, 128x128 with
+    K split, 128x128 unsplit) or, at 512 x 16384, 128x256 tiles of the
+    eight-wave kernel; every output against the exact oracle (computed once per shape, reused
     under every launch shape)."""
     import joyomni_ops as jo
     a, w, sa, sb, bias = operands(M, N, K, M * 7 + K)
@@ -168,6 +168,19 @@ def test_fp8_scaled_mm_text_stream_shapes(dev, M, N, K):
     err = (out.cpu().double() - ref).abs()
     bad = (err > tol).nonzero()
     assert bad.numel() == 0, f"[{M},{N},{K}]: {bad.shape[0]} outputs off, first {bad[0].tolist()}"
+
+
+@pytest.mark.parametrize("sb_at,bias_at", [(1, 0), (0, 1), (0, 2), (3, 3)])
+@pytest.mark.parametrize("M,N,K", [(200, 136, 336), (20, 4104, 256)])
+def test_fp8_scaled_mm_misaligned_scales_and_bias(dev, M, N, K, sb_at, bias_at):
+    """scales_b or bias that does not start on 16 or 8 bytes: the register-staged
+    kernel, whatever the shape would otherwise take."""
+    import joyomni_ops as jo
+    a, w, sa, sb, bias = operands(M, N, K, M + sb_at + bias_at)
+    sbd = torch.cat([torch.full((sb_at,), float("nan")), sb]).to(dev)[sb_at:]
+    bd = torch.cat([torch.full((bias_at,), float("nan")).to(bias.dtype), bias]).to(dev)[bias_at:]
+    out = jo.fp8_scaled_mm(a.to(dev), w.to(dev).t(), sa.to(dev), sbd, torch.bfloat16, bd)
+    check(out, a, w.t(), sa, sb, bias, f"[{M},{N},{K}] scales_b + {sb_at}, bias + {bias_at}")
 
 
 @pytest.mark.parametrize("split", [2, 4, 8])
