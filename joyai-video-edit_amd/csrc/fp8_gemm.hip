@@ -7,15 +7,14 @@
 // reference's visitor tree (fp8_gemm.cu:99-136: acc * scale_b, then
 // scale_a * that + bias, round to nearest).
 //
-// gfx950 design: one 256-thread workgroup per 256x256 output tile; the four
-// waves own 128x128 quadrants computed with v_mfma_f32_32x32x64_f8f6f4
-// (4x4 MFMA tiles, 256 fp32 accumulators per lane). K advances in 128-byte
-// stages: every thread loads 8 sixteen-byte chunks of A and 8 of B^T from
-// HBM into registers for the next stage while the MFMAs run on the current
-// one, then writes them to the other half of a double-buffered LDS tile
-// (2 x 64 KB). LDS rows are 128 bytes; chunk c of row r is stored at chunk
-// position c ^ (r % 8) ^ ((r / 8) % 2), so the 16 rows a 16-lane group
-// reads with one ds_read_b128 fall in 16 distinct 16-byte bank groups.
+// Four kernels, chosen by plan_gemm from M, N, K and the CU count:
+//   pair    many rows: eight waves on a tile of 96 to 256 rows x 256 columns;
+//   small   a few hundred rows: tiles of 64x64 to 128x192, with split K for few
+//           tiles and a long K;
+//   stream  up to 80 rows: all of them by 16 to 64 columns, the waves sharing K;
+//   staged  what the others' direct global->LDS loads do not take: K == 0,
+//           scales_b not 16-byte or bias not 8-byte aligned, 256 operand rows of
+//           4 GiB and more.
 
 #include <atomic>
 #include <type_traits>
@@ -62,6 +61,15 @@ __device__ __forceinline__ f32x4 mfma16(const i32x8& a, const i32x8& b, const f3
   return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, c, 0, 0, 0, 0, 0, 0);
 }
 
+// Staged kernel: one 256-thread workgroup per 256x256 output tile; the four
+// waves own 128x128 quadrants computed with v_mfma_f32_32x32x64_f8f6f4
+// (4x4 MFMA tiles, 256 fp32 accumulators per lane). K advances in 128-byte
+// stages: every thread loads 8 sixteen-byte chunks of A and 8 of B^T from
+// HBM into registers for the next stage while the MFMAs run on the current
+// one, then writes them to the other half of a double-buffered LDS tile
+// (2 x 64 KB). LDS rows are 128 bytes; chunk c of row r is stored at chunk
+// position c ^ (r % 8) ^ ((r / 8) % 2), so the 16 rows a 16-lane group
+// reads with one ds_read_b128 fall in 16 distinct 16-byte bank groups.
 template <class OutTag>
 __global__ __launch_bounds__(kBlock, 1) void fp8_gemm_kernel(const GemmArgs g) {
   __shared__ __attribute__((aligned(16))) uint8_t smem[2 * kStageBytes];  // 2 stages
@@ -209,15 +217,19 @@ __device__ __forceinline__ void wait_loads(int later) {
 //                         | s+1's first fragments into registers set free
 // so every fragment register is loaded under MFMAs that do not need it.
 // LDS rows are 128 bytes; chunk c of row r sits at chunk position
-// c ^ ((r >> 1) & 7): the sixteen consecutive rows a 16-lane group reads with
-// one ds_read_b128 then fall in sixteen distinct 16-byte bank groups.
+// c ^ ((r >> 1) & 7): the sixteen consecutive rows that lanes 0-15 read with one
+// ds_read_b128 fall in sixteen distinct 16-byte bank groups. (The bank-conflict
+// counter still stands at half of the LDS cycles, where the 32-row fragments of
+// 32x32x64 in this layout count next to none.)
 //
-// What bounds it is power: with random operands the MFMAs alone (from
-// registers, no memory) run at 4.0 PFLOP/s, the clock falling to ~1.95 GHz,
-// and at 3.7 with 32x32x64, whose accumulators move twice the bits per flop. A
-// 208-row stage takes ~2050 cycles for 1664 of MFMAs at 1.85-1.95 GHz, and
-// forms with fewer idle cycles run at lower clocks for the same time (four
-// waves of 128 x 128, with a third less LDS traffic: 2-12% slower). Measured
+// What bounds it is power first: the same launches on zero operands take
+// 101.1 us for 124.0 at 3120x12288x4096, 121.3 for 147.9 at 3120x4096x16384, and
+// the clock of the counter runs is about 1.9 GHz there, of 2.4. From registers
+// alone, on random operands, 16x16x128 reaches 4.6 PFLOP/s at 2.26 GHz and
+// 32x32x64, whose accumulators move twice the bits per flop, 4.2 at 2.04 (5.0 at
+// 2.39 both on zeros); the matrix cores are busy for 0.55 to 0.61 of this
+// kernel's cycles. Four waves of 128 x 128, with a third less LDS traffic,
+// measured 2-12% slower. Measured
 // against the same tiles on 32x32x64 with 224 or 256 rows only:
 // 3120x12288x4096 130 -> 123.5 us, 3120x16384x4096 173 -> 162,
 // 3120x4096x16384 168 -> 164, 3120x4096x4096 45 -> 41.5, 4096^3 55 -> 52,
@@ -574,30 +586,36 @@ __device__ __forceinline__ void fp8_gemm_pair_tile(const GemmArgs& g, uint8_t* s
   // Rows that do not start on a line (N of no multiple of 64): a wave's pieces
   // then end inside lines that the next wave completes, so they are left to the
   // L2 to join instead of written through: us, through / joined, 4326x10968x640
-  // 60.8 / 42.8, 4066x4072x128 14.6 / 10.7, 3184x9384x1280 52.1 / 44.6, 2815x5128x6144
-  // 76.6 / 72.6. Whole lines written through are not read again and stay out of
-  // the L2.
+  // 57.7 / 40.7, 4066x4072x128 14.6 / 10.7, 3184x9384x1280 52.3 / 44.0. Whole lines
+  // written through are not read again and stay out of the L2. A copy of the loop
+  // for each: with the choice inside it 3120x4096x4096 took 43.8 us for 42.7.
   const bool whole_lines = g.ldo % 64 == 0 && (reinterpret_cast<uintptr_t>(g.out) & 127) == 0;
   // A wave's LDS operations run in order, so block i's reads follow its
   // writes; block i + 1 is written before block i leaves.
-  stage_block(0);
+  auto leave = [&](auto lines) {
+    stage_block(0);
 #pragma unroll
-  for (int i = 0; i < MI; ++i) {
-    if (i + 1 < MI) stage_block(i + 1);
-    asm volatile("" ::: "memory");
+    for (int i = 0; i < MI; ++i) {
+      if (i + 1 < MI) stage_block(i + 1);
+      asm volatile("" ::: "memory");
 #pragma unroll
-    for (int r = i * 16; r < i * 16 + 16; r += kRowsPerStore) {
-      const int m = m0 + row0 + r + sr, n = n0 + wn * WCOLS + sc * 8;
-      const u32x4 v = *reinterpret_cast<const u32x4*>(mine + (r + sr) * kRowBytes + sc * 16);
-      if (m < g.M && n < g.N) {
-        uint16_t* dst = static_cast<uint16_t*>(g.out) + static_cast<int64_t>(m) * g.ldo + n;
-        if (whole_lines)
-          st16_nt(dst, v);
-        else
-          st16(dst, v);
+      for (int r = i * 16; r < i * 16 + 16; r += kRowsPerStore) {
+        const int m = m0 + row0 + r + sr, n = n0 + wn * WCOLS + sc * 8;
+        const u32x4 v = *reinterpret_cast<const u32x4*>(mine + (r + sr) * kRowBytes + sc * 16);
+        if (m < g.M && n < g.N) {
+          uint16_t* dst = static_cast<uint16_t*>(g.out) + static_cast<int64_t>(m) * g.ldo + n;
+          if constexpr (decltype(lines)::value)
+            st16_nt(dst, v);
+          else
+            st16(dst, v);
+        }
       }
     }
-  }
+  };
+  if (whole_lines)
+    leave(T{});
+  else
+    leave(F{});
 }
 
 // Output tile of this workgroup. The dispatcher hands workgroup id (linear
@@ -707,15 +725,15 @@ void launch_pair_rows(const GemmArgs& g, hipStream_t stream, int rows) {
 }
 
 // ---------------------------------------------------------------------------
-// Small-tile kernel, for grids the 8-wave 224/256-row tiles would leave
-// mostly idle (a few hundred rows: the text stream's Fp8Linear calls; 224x256
-// tiles give [256, 4096] 32 tiles for 256 CUs). NW waves on a BM x BN tile
-// (64x64, 64x128, 128x128 or 128x192 with four, 128x256 with eight) in a
-// WGM x NW/WGM grid of wave tiles (WGM = 2); the 96-column tiles give each
-// wave 32 x 96 (128x96: four waves down the rows, WGM = 4; 64x96: two waves,
-// WGM = 2, two workgroups to a CU's LDS); K advances in 128-byte stages (whole lines, the LDS layout of the
-// 128-byte-stage kernel) through a ring of NST slots that direct loads fill
-// NST-1 stages ahead; one barrier a stage.
+// Small-tile kernel, for grids that the pair kernel's 256-column tiles would
+// leave mostly idle (a few hundred rows: the text stream's Fp8Linear calls;
+// [256, 4096] is 32 tiles of 128x256 for 256 CUs). NW waves on a BM x BN tile
+// (64x64, 64x128, 128x128 or 128x192 with four) in a WGM x NW/WGM grid of wave
+// tiles (WGM = 2); the 96-column tiles give each wave 32 x 96 (128x96: four
+// waves down the rows, WGM = 4; 64x96: two waves, WGM = 2, two workgroups to a
+// CU's LDS); K advances in 128-byte stages (whole lines, the pair kernel's LDS
+// layout) through a ring of NST slots that direct loads fill NST-1 stages ahead;
+// one barrier a stage.
 // Its K loop streams (BM + BN) x 128 bytes a stage for BM x BN x 128 MACs, so
 // it only pays where it brings CUs into play that the large tiles leave idle.
 // ---------------------------------------------------------------------------
@@ -819,7 +837,8 @@ __device__ __forceinline__ void fp8_gemm_small_body(const GemmArgs& g) {
         const u32x4 hi = *reinterpret_cast<const u32x4*>(st + offa[k][1] + i * 32 * kQBK);
         af[i] = i32x8{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
       }
-      // B first: the accumulator is the transposed tile (as in store_tile).
+      // B first: the accumulator is the transposed tile (a lane holds one
+      // output row, four of every eight columns).
 #pragma unroll
       for (int i = 0; i < MI; ++i)
 #pragma unroll
