@@ -1306,18 +1306,23 @@ int auto_shape(int cus, int M, int N, int K) {
 constexpr int64_t kSplitCap = int64_t{1} << 30;  // largest partial buffer a split uses
 
 // Estimated time of the streaming kernel, ns: the launch, first loads and last
-// exchange; the busiest CU's rows of A (70 KB/us) and columns of B (35 KB/us),
-// or B at what HBM gives all CUs (5.3 TB/s) with A beside it, whichever is
-// longer; and what a workgroup and a block of the exchange cost. The constants
-// here and in plan_gemm were fitted so that no choice was slower than the
-// kernel it replaces on 770 shapes (1 to 80 rows, N 512 to 16384, K 512 to
-// 16384), with weights from HBM and with cached ones: each of the four widths
-// measured on each, 0.91 of the time that the best choice saves is saved.
+// exchange; the busiest CU's rows of A (72 KB/us) and columns of B (39 KB/us),
+// or B at what HBM gives all CUs (5.25 TB/s) with a part of A beside it,
+// whichever is longer; what a row block, a workgroup and a block of the exchange
+// cost; and, with rows a multiple of 8 KB apart, whose lines fall on the same
+// channels, 4 us where narrow tiles keep most CUs at it (64x8192x8192 21.9 us,
+// x6144 14.8). The constants here and in plan_gemm are fitted to 770 shapes (1 to
+// 80 rows, N 512 to 16384, K 512 to 16384), each of the four widths measured on
+// each with the weight from HBM and cached: 0.96 of the time that the best
+// choices save is saved, and four shapes are slower than with the kernel that
+// streaming replaces, by 2-3% (80x8192x4096, x5120 and 64x9216x512) or with a
+// cached weight only (16x3072x16384 13.6 -> 14.8; from HBM 16.5 -> 15.1).
 int64_t stream_ns(int M, int N, int K, int nb) {
   const int64_t tiles = (N + nb * 16 - 1) / (nb * 16);  // at most one a CU
   const int64_t mb = (M + 15) / 16, a = mb * 16 * K, b = static_cast<int64_t>(nb) * 16 * K;
-  const int64_t cu = a / 70 + b / 35, hbm = static_cast<int64_t>(N) * K / 5300 + a / 85;
-  return 3000 + (cu > hbm ? cu : hbm) + 2 * tiles + 40 * mb * nb;
+  const int64_t cu = a / 72 + b / 39, hbm = static_cast<int64_t>(N) * K * 4 / 21000 + a / 200;
+  const int64_t channels = K % 8192 == 0 && mb >= 3 && nb <= 2 && tiles > 192 ? 4000 : 0;
+  return 3000 + (cu > hbm ? cu : hbm) + 150 * mb + tiles + 36 * mb * nb + channels;
 }
 
 struct GemmPlan {
@@ -1384,19 +1389,21 @@ GemmPlan plan_gemm(const GemmArgs& g, int64_t ws_bytes) {
   const bool splits = best >= 0 && best * 20 < unsplit * 17;
   if (splits) p = split;
   // Few rows: the streaming kernel where it is estimated faster than the
-  // choice so far: 3.6 us and its operand bytes at 52 KB/us a CU (3 us more for
-  // the two waves of 64x96 tiles); with a split 10.5 us for the two launches and
-  // 100 KB/us, or 30 where workgroups share a CU (streaming was faster on every
-  // such shape). A weight that comes from HBM decides most of them: 80x2048x6144
-  // 10.6 us split in four, 12.3 streamed (cached 9.5 and 7.1). Only where one
-  // round of workgroups takes all columns: past that the short K's measured up
-  // to half slower (57x17632x128 5.1 -> 7.6).
+  // choice so far: 4.25 us and its operand bytes at 54 KB/us a CU (59 with two
+  // tile rows), or the weight at 5.3 TB/s; 1 us more for the two waves of 64x96
+  // tiles; with a split 10 us for the two launches and 75 KB/us, or 30 where
+  // workgroups share a CU (streaming was faster on every such shape). A weight
+  // that comes from HBM decides most of them: 80x2048x6144 10.6 us split in four,
+  // 12.3 streamed (cached 9.5 and 7.1). Only where one round of workgroups takes
+  // all columns: past that the short K's measured up to half slower
+  // (57x17632x128 5.1 -> 7.6).
   if (g.M <= kStreamRows) {
-    int64_t other = 3600 + unsplit / 52 + (p.shape == 11 ? 3000 : 0);
+    const int64_t draw = unsplit / (g.M > 64 ? 59 : 54), weight = static_cast<int64_t>(g.N) * g.K / 5300;
+    int64_t other = 4250 + (draw > weight ? draw : weight) + (p.shape == 11 ? 1000 : 0);
     if (splits) {
       const int64_t t = split.shape == 5 ? 128 : 64;
       const int64_t wgs = (g.M + t - 1) / t * ((g.N + t - 1) / t) * split.splits, per = (wgs + cus - 1) / cus;
-      other = 10500 + per * 2 * t * (g.K / split.splits) / (per > 1 ? 30 : 100);
+      other = 10000 + per * 2 * t * (g.K / split.splits) / (per > 1 ? 30 : 75);
     }
     for (int nb = 1; nb <= 4; ++nb) {
       if (g.N > cus * nb * 16 || !stream_built((g.M + 15) / 16, nb)) continue;

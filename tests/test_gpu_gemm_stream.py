@@ -34,16 +34,16 @@ def test_few_rows(dev, M, N, K, dtype):
 
 # (row blocks, column blocks): (N, K) that select them on 256 CUs.
 WIDTHS = {
-    (1, 1): [(8, 16), (24, 1040)], (1, 2): [(760, 16), (3992, 1040)],
-    (1, 3): [(2248, 16), (6952, 1040)], (1, 4): [(4664, 16), (9608, 1040)],
-    (2, 1): [(8, 16), (24, 1040)], (2, 2): [(1400, 16), (4104, 1040)],
-    (2, 3): [(4168, 16), (7336, 1040)], (2, 4): [(8296, 16), (10008, 1040)],
-    (3, 1): [(8, 16), (24, 1040)], (3, 2): [(2040, 16), (4104, 1040)],
-    (3, 3): [(7320, 272), (7720, 1040)],
-    (4, 1): [(8, 16), (24, 1040)], (4, 2): [(2680, 16), (4104, 1040)],
-    (4, 3): [(8104, 2048), (8104, 2320)],
-    (5, 1): [(8, 16), (24, 1040)], (5, 2): [(4104, 272), (4104, 1040)],
-    (5, 3): [(8200, 16), (8200, 1040)], (5, 4): [(12296, 2048), (12296, 2320)],
+    (1, 1): [(8, 16), (24, 1040)], (1, 2): [(2008, 16), (4104, 1040)],
+    (1, 3): [(6008, 16), (8200, 1040)], (1, 4): [(12296, 16), (12296, 1040)],
+    (2, 1): [(8, 16), (24, 1040)], (2, 2): [(4104, 16), (4104, 1040)],
+    (2, 3): [(8200, 16), (8200, 1040)], (2, 4): [(12296, 16), (12296, 1040)],
+    (3, 1): [(8, 16), (24, 1040)], (3, 2): [(4104, 16), (4104, 1040)],
+    (3, 3): [(8200, 16), (8200, 1040)],
+    (4, 1): [(8, 16), (24, 1040)], (4, 2): [(4104, 16), (4104, 1040)],
+    (4, 3): [(8200, 16), (8200, 1040)],
+    (5, 1): [(8, 16), (24, 1040)], (5, 2): [(4104, 16), (4104, 1040)],
+    (5, 3): [(8200, 16), (8200, 1040)], (5, 4): [(12296, 1040), (12296, 2320)],
 }
 
 
