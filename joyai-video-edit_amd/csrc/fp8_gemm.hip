@@ -229,12 +229,11 @@ __device__ __forceinline__ void wait_loads(int later) {
 // 32x32x64, whose accumulators move twice the bits per flop, 4.2 at 2.04 (5.0 at
 // 2.39 both on zeros); the matrix cores are busy for 0.55 to 0.61 of this
 // kernel's cycles. Four waves of 128 x 128, with a third less LDS traffic,
-// measured 2-12% slower. Measured
-// against the same tiles on 32x32x64 with 224 or 256 rows only:
-// 3120x12288x4096 130 -> 123.5 us, 3120x16384x4096 173 -> 162,
-// 3120x4096x16384 168 -> 164, 3120x4096x4096 45 -> 41.5, 4096^3 55 -> 52,
-// 8192^3 408 -> 393 (2.8 PFLOP/s), 1560x12288x4096 80.5 -> 67,
-// 1560x4096x4096 32 -> 26, 512x12288x4096 30.7 -> 26.7.
+// measured 2-12% slower. Against the same tiles on 32x32x64 with 224 or 256 rows
+// only, us, weights from HBM: 3120x12288x4096 130.4 -> 126.7, 3120x16384x4096 174.0
+// -> 165.6, 3120x4096x16384 158.7 -> 153.9, 3120x4096x4096 45.5 -> 43.3, 4096^3 53.6
+// -> 52.2, 1560x12288x4096 91.9 -> 67.3, 1560x4096x4096 32.8 -> 28.8, 512x12288x4096
+// 32.0 -> 31.4 (cached 31.5 -> 26.2).
 // ---------------------------------------------------------------------------
 constexpr int kQBK = 128;  // bytes of K per stage
 
@@ -1025,11 +1024,11 @@ void launch_small(const GemmArgs& g, hipStream_t stream, int splits = 1) {
 // waves' loads are in flight meanwhile. The partial tiles meet in LDS at the
 // end and are added in wave order (the same bits on every run).
 // Measured against the small-tile kernel, us, weights from HBM / cached:
-// 16x4096x4096 11.7 -> 6.8 (HBM), 40x4096x4096 12.2 -> 8.3, 77x4096x4096 12.1
-// -> 10.2 / 10.4 -> 8.3, 77x12288x4096 17.4 -> 16.9 / 15.8 -> 12.3,
-// 77x16384x4096 19.2 -> 20.3 / 15.5 -> 14.9 (left to it), 1x12288x4096 13.3 -> 11.7 /
-// 10.3 -> 9.9, 24x3072x3072 9.9 -> 5.6 / 8.3 -> 3.9. About 4 us of it are the launch, the first loads' latency and the
-// last exchange; at 77 rows every workgroup also reads 320 KB of A from its L2.
+// 1x4096x4096 11.4 -> 6.8 / 10.0 -> 4.0, 40x4096x4096 11.9 -> 7.8 / 10.1 -> 5.9,
+// 77x4096x4096 11.5 -> 9.7 / 10.1 -> 7.7, 77x12288x4096 16.8 -> 15.2 / 16.0 -> 12.4,
+// 1x12288x4096 13.5 -> 11.8 / 10.7 -> 9.3, 24x3072x3072 9.5 -> 5.4 / 8.2 -> 3.6.
+// About 4 us of it are the launch, the first loads' latency and the last
+// exchange; at 77 rows every workgroup also reads 320 KB of A from its L2.
 // Fragments loaded straight into registers in MFMA layout (64 bytes a row and
 // load instead of whole lines) measured 20.4 / 17.8 at 77x12288x4096;
 // nontemporal loads of B 14.9 / 14.3 (77x16384x4096 18.2 / 17.7): nothing of the
@@ -1038,6 +1037,9 @@ void launch_small(const GemmArgs& g, hipStream_t stream, int splits = 1) {
 constexpr int kStreamLds = 152 * 1024;
 
 constexpr int kStreamWaves = 8;
+// Five row blocks: what four column blocks leave room for in LDS. Up to 128 rows
+// would fit with fewer columns; between 81 and 127 that is not measured, 128 rows
+// were slower.
 constexpr int kStreamRows = 80;
 
 template <int MB, int NB>
