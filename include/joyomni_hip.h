@@ -423,11 +423,11 @@ int jo_fp8_scaled_mm(const void* mat_a, int64_t lda, const void* mat_b, int64_t 
  * several workgroups per tile, which write fp32 partial products to the
  * workspace that a second kernel adds up in a fixed order: results are the
  * same on every run, and equal to jo_fp8_scaled_mm's up to fp32 summation
- * order. A workspace smaller than jo_fp8_scaled_mm_workspace_bytes(M, N, K)
- * (NULL with 0 bytes included) runs exactly as jo_fp8_scaled_mm. The
- * workspace is in use until the work queued on `stream` finishes; two calls
- * in flight at once need two workspaces. The torch op fp8_scaled_mm takes
- * it from the caching allocator. Reference counterpart: the same
+ * order. With a workspace smaller than jo_fp8_scaled_mm_workspace_bytes(M, N, K)
+ * K is split as far as it has room for and that pays, and with none (NULL, 0
+ * bytes) the call runs exactly as jo_fp8_scaled_mm. The workspace is in use
+ * until the work queued on `stream` finishes; two calls in flight at once need
+ * two workspaces. The torch op fp8_scaled_mm takes it from the caching allocator. Reference counterpart: the same
  * fp8_scaled_mm (fp8_gemm.cu:1450-1546), whose CUTLASS kernel allocates its
  * own workspace. */
 int jo_fp8_scaled_mm_ws(const void* mat_a, int64_t lda, const void* mat_b, int64_t ldb,
