@@ -297,7 +297,7 @@ constexpr int pair_ring_bytes() {
 // The K loop and epilogue of a wave holding MI row blocks of 16 (from the
 // tile's row row0 on). NBS: B stages go through a ring of NBS slots beside A's
 // two, so B loads run NBS - 1 stages ahead and A loads one.
-template <class OutTag, int BM, int BN, int NW, int MI, int NBS>
+template <class OutTag, int BM, int BN, int NW, int MI, int NBS, bool LINES>
 __device__ __forceinline__ void fp8_gemm_pair_tile(const GemmArgs& g, uint8_t* smem,
                                                    const PairLoads<BM, BN, NW>& ld, const KTail& kt, int wave,
                                                    int row0, int wn, int m0, int n0) {
@@ -582,39 +582,33 @@ __device__ __forceinline__ void fp8_gemm_pair_tile(const GemmArgs& g, uint8_t* s
       *reinterpret_cast<u32x2*>(mine + (i * 16 + fr) * kRowBytes + (j * 16 + fh * 4) * 2) = u32x2{pk.x, pk.y};
     }
   };
-  // Rows that do not start on a line (N of no multiple of 64): a wave's pieces
-  // then end inside lines that the next wave completes, so they are left to the
-  // L2 to join instead of written through: us, through / joined, 4326x10968x640
-  // 57.7 / 40.7, 4066x4072x128 14.6 / 10.7, 3184x9384x1280 52.3 / 44.0. Whole lines
-  // written through are not read again and stay out of the L2. A copy of the loop
-  // for each: with the choice inside it 3120x4096x4096 took 43.8 us for 42.7.
-  const bool whole_lines = g.ldo % 64 == 0 && (reinterpret_cast<uintptr_t>(g.out) & 127) == 0;
+  // LINES: output rows start on 128-byte lines. Where they do not (N of no multiple
+  // of 64) a wave's pieces end inside lines that the next wave completes, so they
+  // are left to the L2 to join instead of written through: us, through / joined,
+  // 4326x10968x640 57.7 / 40.7, 4066x4072x128 14.6 / 10.7, 3184x9384x1280 52.3 / 44.0.
+  // Whole lines written through are not read again and stay out of the L2. A
+  // kernel for each: with the choice in this loop 3120x4096x4096 took 43.8 us for
+  // 42.7, with a copy of the loop for each behind another kernel 51.0 for 50.4.
   // A wave's LDS operations run in order, so block i's reads follow its
   // writes; block i + 1 is written before block i leaves.
-  auto leave = [&](auto lines) {
-    stage_block(0);
+  stage_block(0);
 #pragma unroll
-    for (int i = 0; i < MI; ++i) {
-      if (i + 1 < MI) stage_block(i + 1);
-      asm volatile("" ::: "memory");
+  for (int i = 0; i < MI; ++i) {
+    if (i + 1 < MI) stage_block(i + 1);
+    asm volatile("" ::: "memory");
 #pragma unroll
-      for (int r = i * 16; r < i * 16 + 16; r += kRowsPerStore) {
-        const int m = m0 + row0 + r + sr, n = n0 + wn * WCOLS + sc * 8;
-        const u32x4 v = *reinterpret_cast<const u32x4*>(mine + (r + sr) * kRowBytes + sc * 16);
-        if (m < g.M && n < g.N) {
-          uint16_t* dst = static_cast<uint16_t*>(g.out) + static_cast<int64_t>(m) * g.ldo + n;
-          if constexpr (decltype(lines)::value)
-            st16_nt(dst, v);
-          else
-            st16(dst, v);
-        }
+    for (int r = i * 16; r < i * 16 + 16; r += kRowsPerStore) {
+      const int m = m0 + row0 + r + sr, n = n0 + wn * WCOLS + sc * 8;
+      const u32x4 v = *reinterpret_cast<const u32x4*>(mine + (r + sr) * kRowBytes + sc * 16);
+      if (m < g.M && n < g.N) {
+        uint16_t* dst = static_cast<uint16_t*>(g.out) + static_cast<int64_t>(m) * g.ldo + n;
+        if constexpr (LINES)
+          st16_nt(dst, v);
+        else
+          st16(dst, v);
       }
     }
-  };
-  if (whole_lines)
-    leave(T{});
-  else
-    leave(F{});
+  }
 }
 
 // Output tile of this workgroup. The dispatcher hands workgroup id (linear
@@ -639,7 +633,7 @@ __device__ __forceinline__ void xcd_grouped_tile(int group, int bm, int bn, int&
   n0 = (w / rows) * bn;
 }
 
-template <class OutTag, int BM, int BN, int NW, int NBS>
+template <class OutTag, int BM, int BN, int NW, int NBS, bool LINES>
 __device__ __forceinline__ void fp8_gemm_pair_body(const GemmArgs& g) {
   using Loads = PairLoads<BM, BN, NW>;
   constexpr int RB = BM / 16;  // 16-row blocks: the first wave row takes (RB + 1) / 2
@@ -674,18 +668,18 @@ __device__ __forceinline__ void fp8_gemm_pair_body(const GemmArgs& g) {
   ld.last = Loads::kEven || wave + (Loads::kPerWave - 1) * NW < Loads::kSlots;
   constexpr int kUp = (RB + 1) / 2, kLow = RB / 2;
   if constexpr (kUp == kLow) {
-    fp8_gemm_pair_tile<OutTag, BM, BN, NW, kUp, NBS>(g, smem, ld, kt, wave, wm * kUp * 16, wn, m0, n0);
+    fp8_gemm_pair_tile<OutTag, BM, BN, NW, kUp, NBS, LINES>(g, smem, ld, kt, wave, wm * kUp * 16, wn, m0, n0);
   } else {
     if (wm == 0)
-      fp8_gemm_pair_tile<OutTag, BM, BN, NW, kUp, NBS>(g, smem, ld, kt, wave, 0, wn, m0, n0);
+      fp8_gemm_pair_tile<OutTag, BM, BN, NW, kUp, NBS, LINES>(g, smem, ld, kt, wave, 0, wn, m0, n0);
     else
-      fp8_gemm_pair_tile<OutTag, BM, BN, NW, kLow, NBS>(g, smem, ld, kt, wave, kUp * 16, wn, m0, n0);
+      fp8_gemm_pair_tile<OutTag, BM, BN, NW, kLow, NBS, LINES>(g, smem, ld, kt, wave, kUp * 16, wn, m0, n0);
   }
 }
 
-template <class OutTag, int BM, int BN, int NW, int NBS>
+template <class OutTag, int BM, int BN, int NW, int NBS, bool LINES>
 __global__ __launch_bounds__(NW * 64, 1) void fp8_gemm_pair_kernel(const GemmArgs g) {
-  fp8_gemm_pair_body<OutTag, BM, BN, NW, NBS>(g);
+  fp8_gemm_pair_body<OutTag, BM, BN, NW, NBS, LINES>(g);
 }
 
 // Tile rows of a group of xcd_grouped_tile: equal groups of at most five (six
@@ -704,8 +698,11 @@ template <class OutTag, int BM, int BN, int NW, int NBS>
 void launch_pair(const GemmArgs& args, hipStream_t stream) {
   GemmArgs g = args;
   g.group = group_rows((g.M + BM - 1) / BM);
-  hipLaunchKernelGGL((fp8_gemm_pair_kernel<OutTag, BM, BN, NW, NBS>),
-                     dim3((g.N + BN - 1) / BN, (g.M + BM - 1) / BM), dim3(NW * 64), 0, stream, g);
+  const dim3 grid((g.N + BN - 1) / BN, (g.M + BM - 1) / BM);
+  if (g.ldo % 64 == 0 && aligned(g.out, 128))
+    hipLaunchKernelGGL((fp8_gemm_pair_kernel<OutTag, BM, BN, NW, NBS, true>), grid, dim3(NW * 64), 0, stream, g);
+  else
+    hipLaunchKernelGGL((fp8_gemm_pair_kernel<OutTag, BM, BN, NW, NBS, false>), grid, dim3(NW * 64), 0, stream, g);
 }
 
 // The pair kernel at `rows` tile rows (a multiple of 16 from 96 to 256), B two
