@@ -222,13 +222,13 @@ __device__ __forceinline__ void wait_loads(int later) {
 // counter still stands at half of the LDS cycles, where the 32-row fragments of
 // 32x32x64 in this layout count next to none.)
 //
-// What bounds it is power first: the same launches on zero operands take
-// 101.1 us for 124.0 at 3120x12288x4096, 121.3 for 147.9 at 3120x4096x16384, and
-// the clock of the counter runs is about 1.9 GHz there, of 2.4. From registers
-// alone, on random operands, 16x16x128 reaches 4.6 PFLOP/s at 2.26 GHz and
-// 32x32x64, whose accumulators move twice the bits per flop, 4.2 at 2.04 (5.0 at
-// 2.39 both on zeros); the matrix cores are busy for 0.55 to 0.61 of this
-// kernel's cycles. Four waves of 128 x 128, with a third less LDS traffic,
+// What bounds it: idle matrix cores (busy for 0.46 to 0.62 of the cycles at
+// 3120 rows: epilogues, rounds, the first stages) and the clock, which power holds
+// at 1.9-2.1 GHz of 2.4: the same launches on zero operands take 102.7 us for
+// 120.7 at 3120x12288x4096, 119.9 for 143.7 at 3120x4096x16384. From registers
+// alone, on random operands, 16x16x128 reaches 4.5-4.6 PFLOP/s at 2.2 GHz and
+// 32x32x64, whose accumulators move twice the bits per flop, 4.1-4.2 at 2.0 (5.0
+// at 2.4 both on zeros). Four waves of 128 x 128, with a third less LDS traffic,
 // measured 2-12% slower. Against the same tiles on 32x32x64 with 224 or 256 rows
 // only, us, weights from HBM: 3120x12288x4096 130.4 -> 126.7, 3120x16384x4096 174.0
 // -> 165.6, 3120x4096x16384 158.7 -> 153.9, 3120x4096x4096 45.5 -> 43.3, 4096^3 53.6
