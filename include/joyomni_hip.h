@@ -427,9 +427,9 @@ int jo_fp8_scaled_mm(const void* mat_a, int64_t lda, const void* mat_b, int64_t 
  * K is split as far as it has room for and that pays, and with none (NULL, 0
  * bytes) the call runs exactly as jo_fp8_scaled_mm. The workspace is in use
  * until the work queued on `stream` finishes; two calls in flight at once need
- * two workspaces. The torch op fp8_scaled_mm takes it from the caching allocator. Reference counterpart: the same
- * fp8_scaled_mm (fp8_gemm.cu:1450-1546), whose CUTLASS kernel allocates its
- * own workspace. */
+ * two workspaces. The torch op fp8_scaled_mm takes it from the caching
+ * allocator. Reference counterpart: the same fp8_scaled_mm
+ * (fp8_gemm.cu:1450-1546), whose CUTLASS kernel allocates its own workspace. */
 int jo_fp8_scaled_mm_ws(const void* mat_a, int64_t lda, const void* mat_b, int64_t ldb,
                         const float* scales_a, const float* scales_b, const void* bias, void* out,
                         int64_t ldo, int64_t M, int64_t N, int64_t K, int out_dtype,
